@@ -3,11 +3,10 @@
 // Reference: QuantizedLinear::quantize / dequantize_weight
 // (src/primitives/quant.rs:38-53, :73-81) -> mlx_rs::ops::{quantize,dequantize}
 // (MLX 0.31.2); the per-group arithmetic is in affine_group.hpp.
-// Layout: every lane owns 8 consecutive elements; the group_size/8 lanes of a
-// group reduce min/max with butterfly shuffles, then each lane packs its own
-// codes into one (Q4) or two (Q8) uint32 words, so loads and stores are fully
-// coalesced 16-byte accesses.  This file is compiled with -ffp-contract=off:
-// codes must be bit-identical with the CPU restatement.
+// Layout: every lane owns 8 (f32) or 16 (bf16) consecutive elements; the lanes
+// of a group reduce min/max with lane moves, then each lane packs its own
+// codes into whole uint32 words.  This file is compiled with
+// -ffp-contract=off: codes must be bit-identical with the CPU restatement.
 #include <hip/hip_runtime.h>
 
 #include <string>
@@ -19,25 +18,22 @@ namespace mlxq {
 namespace {
 
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 
 constexpr int kThreads = 256;
 
-template <int DT>
-__device__ __forceinline__ void load8(const void* w, int64_t e, float (&v)[8]) {
-  if constexpr (DT == MLXQ_F32) {
-    const float4* p = reinterpret_cast<const float4*>(static_cast<const float*>(w) + e);
-    float4 a = p[0], b = p[1];
-    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-  } else {
-    uint4 u = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(w) + e);
-    uint32_t s[4] = {u.x, u.y, u.z, u.w};
+// EPL consecutive elements (16-byte loads)
+template <int DT, int EPL>
+__device__ __forceinline__ void load_elems(const void* w, int64_t lane, float (&v)[EPL]) {
+  constexpr int P = EPL * (DT == MLXQ_F32 ? 4 : 2) / 16;
+  u32x4 p[P];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      v[2 * i] = bf16_bits_to_f32(s[i] & 0xFFFFu);
-      v[2 * i + 1] = bf16_bits_to_f32(s[i] >> 16);
-    }
+  for (int i = 0; i < P; i++) p[i] = reinterpret_cast<const u32x4*>(w)[lane * P + i];
+#pragma unroll
+  for (int i = 0; i < EPL; i++) {
+    if constexpr (DT == MLXQ_F32) v[i] = bits_to_f32(p[i >> 2][i & 3]);
+    else v[i] = bits_to_f32((i & 1) ? p[i >> 3][(i >> 1) & 3] & 0xFFFF0000u : p[i >> 3][(i >> 1) & 3] << 16);
   }
 }
 
@@ -53,26 +49,31 @@ __device__ __forceinline__ float load1(const void* p, int64_t i) {
   else return bf16_bits_to_f32(static_cast<const uint16_t*>(p)[i]);
 }
 
-// One lane per 8 elements; LPG = group_size / 8 lanes per group.
-template <int DT, int BITS, int LPG>
+// One lane per EPL elements, LPG lanes per group.  Bound by HBM (bf16 in,
+// Q4 out: 2.6 bytes per element) once the per-group arithmetic is shared by
+// enough elements: every lane of a group repeats it, so bf16 takes 16
+// elements per lane (14336 x 4096, Q4 / Q8: 45.9 / 45.8 us with 8 elements
+// and the general division, 36.3 / 37.5 with the shorter quotient, 29.6 /
+// 33.1 = 5.1 / 5.4 TB/s with 16).  f32 input is bound by its loads and takes
+// 8 (Q4 51 -> 47.9 us; 49.7 with 16, whose loads cover a quarter of each
+// line per instruction).  Two and four runs of lanes per workgroup measured
+// slower (bf16 Q4 30.9, f32 Q4 51.3 us with two).
+template <int DT, int BITS, int LPG, int EPL>
 __global__ __launch_bounds__(kThreads) void affine_quantize_kernel(const void* __restrict__ w, int64_t n_lanes,
                                                                     uint32_t* __restrict__ wq,
                                                                     void* __restrict__ scales,
                                                                     void* __restrict__ biases) {
+  constexpr int W = EPL * BITS / 32;  // words per lane
   const int64_t lane = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  const bool active = lane < n_lanes;
-  float v[8];
-  if (active) {
-    load8<DT>(w, lane * 8, v);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = 0.f;
-  }
-  uint32_t codes[8];
+  float v[EPL];
+  load_elems<DT, EPL>(w, min(lane, n_lanes - 1), v);  // clamped: no branch around the load
+  uint32_t words[W];
   float scale, bias;
-  quantize_group8<BITS, LPG>(v, codes, scale, bias);
-  if (!active) return;
-  store_codes8<BITS>(wq, lane, codes);
+  quantize_group<BITS, LPG, EPL>(v, words, scale, bias);  // n_lanes is a multiple of LPG: a group's lanes are all real or all clamped
+  if (lane >= n_lanes) return;
+  if constexpr (W == 1) wq[lane] = words[0];
+  else if constexpr (W == 2) reinterpret_cast<uint2*>(wq)[lane] = make_uint2(words[0], words[1]);
+  else reinterpret_cast<uint4*>(wq)[lane] = make_uint4(words[0], words[1], words[2], words[3]);
   if ((threadIdx.x & (LPG - 1)) == 0) {
     const int64_t g = lane / LPG;
     store1<DT>(scales, g, scale);
@@ -141,12 +142,14 @@ int check_args(int dtype, int64_t rows, int64_t cols, int group_size, int bits) 
 }
 
 template <int DT, int BITS>
-void launch_quant(const void* w, int64_t n_lanes, int group_size, uint32_t* wq, void* s, void* b, hipStream_t st) {
-  dim3 grid(ceil_div(n_lanes, kThreads));
+void launch_quant(const void* w, int64_t n, int group_size, uint32_t* wq, void* s, void* b, hipStream_t st) {
+  constexpr int EPL = DT == MLXQ_F32 ? 8 : 16;
+  const int64_t lanes = n / EPL;
+  const dim3 grid(ceil_div(lanes, kThreads));
   switch (group_size) {
-    case 32: MLXQ_LAUNCH((affine_quantize_kernel<DT, BITS, 4>), grid, dim3(kThreads), 0, st, w, n_lanes, wq, s, b); break;
-    case 64: MLXQ_LAUNCH((affine_quantize_kernel<DT, BITS, 8>), grid, dim3(kThreads), 0, st, w, n_lanes, wq, s, b); break;
-    default: MLXQ_LAUNCH((affine_quantize_kernel<DT, BITS, 16>), grid, dim3(kThreads), 0, st, w, n_lanes, wq, s, b); break;
+    case 32: MLXQ_LAUNCH((affine_quantize_kernel<DT, BITS, 32 / EPL, EPL>), grid, dim3(kThreads), 0, st, w, lanes, wq, s, b); break;
+    case 64: MLXQ_LAUNCH((affine_quantize_kernel<DT, BITS, 64 / EPL, EPL>), grid, dim3(kThreads), 0, st, w, lanes, wq, s, b); break;
+    default: MLXQ_LAUNCH((affine_quantize_kernel<DT, BITS, 128 / EPL, EPL>), grid, dim3(kThreads), 0, st, w, lanes, wq, s, b); break;
   }
 }
 
@@ -160,16 +163,16 @@ extern "C" int mlxq_quantize(const void* w, int dtype, int64_t rows, int64_t col
   clear_error();
   int rc = check_args(dtype, rows, cols, group_size, bits);
   if (rc) return rc;
-  const int64_t n_lanes = rows * cols / 8;
-  if (n_lanes == 0) return MLXQ_OK;
+  const int64_t n = rows * cols;
+  if (n == 0) return MLXQ_OK;
   if (!w || !wq || !scales || !biases) return fail(MLXQ_ERR_INVALID, "quantize: null pointer");
   hipStream_t st = as_stream(stream);
   if (dtype == MLXQ_F32) {
-    if (bits == 4) launch_quant<MLXQ_F32, 4>(w, n_lanes, group_size, wq, scales, biases, st);
-    else launch_quant<MLXQ_F32, 8>(w, n_lanes, group_size, wq, scales, biases, st);
+    if (bits == 4) launch_quant<MLXQ_F32, 4>(w, n, group_size, wq, scales, biases, st);
+    else launch_quant<MLXQ_F32, 8>(w, n, group_size, wq, scales, biases, st);
   } else {
-    if (bits == 4) launch_quant<MLXQ_BF16, 4>(w, n_lanes, group_size, wq, scales, biases, st);
-    else launch_quant<MLXQ_BF16, 8>(w, n_lanes, group_size, wq, scales, biases, st);
+    if (bits == 4) launch_quant<MLXQ_BF16, 4>(w, n, group_size, wq, scales, biases, st);
+    else launch_quant<MLXQ_BF16, 8>(w, n, group_size, wq, scales, biases, st);
   }
   return check_launch("quantize");
 }

@@ -17,12 +17,33 @@
 namespace mlxq {
 namespace {  // internal linkage: each including file has its own copy
 
+// Correctly rounded x / n for finite x of ordinary magnitude (the quotient's
+// residual is then exact): the quotient estimate and one residual step.  With
+// n = 15 or 255 and r = RN(1/n), and with n = 1 .. 257 and r = v_rcp_f32(n),
+// this equals the f32 division for every mantissa of x (checked over all 2^23
+// of them on gfx950); the compiler's general division is 11 instructions.
+__device__ __forceinline__ float div_by(float x, float n, float r) {
+  const float q = x * r;
+  return fmaf(fmaf(-n, q, x), r, q);
+}
+
+// max / min with the value of another lane of the group, without a zeroed
+// destination for the move (every lane is active)
+template <int CTRL>
+__device__ __forceinline__ float dpp_all(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+
 // Lane owns EPL consecutive elements v of a group of EPL * LPG; the LPG
 // lanes of the group (aligned, within one wavefront) reduce min/max with
-// butterfly shuffles.  Every lane of the group must call it.
+// DPP moves.  Every lane of the group must call it.  `words`: the lane's
+// codes packed LSB-first.
+//
+// What bounds it: VALU work.  Per element: the subtraction, two instructions
+// of quotient, one clamp, one rounding add and one pack.
 template <int BITS, int LPG, int EPL = 8>
-__device__ __forceinline__ void quantize_group8(const float (&v)[EPL], uint32_t (&codes)[EPL], float& scale,
-                                                float& bias) {
+__device__ __forceinline__ void quantize_group(const float (&v)[EPL], uint32_t (&words)[EPL * BITS / 32], float& scale,
+                                               float& bias) {
   float w_max = v[0], w_min = v[0];
 #pragma unroll
   for (int i = 1; i < EPL; i++) {
@@ -30,102 +51,90 @@ __device__ __forceinline__ void quantize_group8(const float (&v)[EPL], uint32_t 
     w_min = fminf(w_min, v[i]);
   }
   // All-reduce within the LPG lanes of this group (groups never straddle a
-  // 16-lane row: LPG is 4, 8 or 16 and the lane index is group-aligned) with
+  // 16-lane row: LPG is 2 .. 16 and the lane index is group-aligned) with
   // DPP moves: quad swaps, then the other quad of 8 (lane i <-> 7 - i), then
   // the other 8 of 16 (i <-> 15 - i).  Exact for max/min in any order.
   static_assert(LPG == 2 || LPG == 4 || LPG == 8 || LPG == 16, "lanes per group");
-  w_max = fmaxf(w_max, dpp_f32<kDppQuadXor1>(w_max));
-  w_min = fminf(w_min, dpp_f32<kDppQuadXor1>(w_min));
+  w_max = fmaxf(w_max, dpp_all<kDppQuadXor1>(w_max));
+  w_min = fminf(w_min, dpp_all<kDppQuadXor1>(w_min));
   if constexpr (LPG >= 4) {
-    w_max = fmaxf(w_max, dpp_f32<kDppQuadXor2>(w_max));
-    w_min = fminf(w_min, dpp_f32<kDppQuadXor2>(w_min));
+    w_max = fmaxf(w_max, dpp_all<kDppQuadXor2>(w_max));
+    w_min = fminf(w_min, dpp_all<kDppQuadXor2>(w_min));
   }
   if constexpr (LPG >= 8) {
-    w_max = fmaxf(w_max, dpp_f32<kDppRowHalfMirror>(w_max));
-    w_min = fminf(w_min, dpp_f32<kDppRowHalfMirror>(w_min));
+    w_max = fmaxf(w_max, dpp_all<kDppRowHalfMirror>(w_max));
+    w_min = fminf(w_min, dpp_all<kDppRowHalfMirror>(w_min));
   }
   if constexpr (LPG >= 16) {
-    w_max = fmaxf(w_max, dpp_f32<kDppRowMirror>(w_max));
-    w_min = fminf(w_min, dpp_f32<kDppRowMirror>(w_min));
+    w_max = fmaxf(w_max, dpp_all<kDppRowMirror>(w_max));
+    w_min = fminf(w_min, dpp_all<kDppRowMirror>(w_min));
   }
 
   constexpr float n_bins = static_cast<float>((1 << BITS) - 1);
+  constexpr int CPW = 32 / BITS;  // codes per word
   const float eps = 1e-7f;
   const bool mask = fabsf(w_min) > fabsf(w_max);
-  scale = fmaxf((w_max - w_min) / n_bins, eps);
-  scale = mask ? scale : -scale;
   const float edge = mask ? w_min : w_max;
-  const float q0 = __builtin_rintf(edge / scale);
+  scale = fmaxf(div_by(w_max - w_min, n_bins, 1.0f / n_bins), eps);
+  scale = mask ? scale : -scale;
+  // rint(fl(x / s)), fl the correctly rounded f32 division, is rint of
+  // fma(x, r1, x r2) with r1 + r2 = 1/s to about 48 bits: the two quotients
+  // can only round apart next to a half-integer, and there they were compared
+  // on gfx950 for every mantissa of s, every half-integer up to 256.5 and the
+  // nine x around their product; the one mantissa that differs (all ones,
+  // x/s next to 0.5) takes the division below.  The comparison carries over
+  // to any scale whose products neither overflow nor lose their residuals: s
+  // is at least 1e-7, and |x| at most 2^60 is tested.
+  auto recip = [](float s, float& r1, float& r2) {
+    const float r0 = __builtin_amdgcn_rcpf(s);
+    r1 = fmaf(fmaf(-s, r0, 1.0f), r0, r0);
+    r2 = fmaf(-s, r1, 1.0f) * r1;
+  };
+  float r1, r2;
+  recip(scale, r1, r2);
+  const float q0 = __builtin_rintf(fmaf(edge, r1, edge * r2));
   bias = 0.f;
   if (q0 != 0.f) {
-    scale = edge / q0;
+    scale = div_by(edge, q0, __builtin_amdgcn_rcpf(q0));  // |q0| <= n_bins + 1
     bias = edge;
   }
-
-  // code = rint(fl((w - bias) / scale)), fl the correctly rounded f32
-  // division.  The compiler's division of d by scale is v_div_scale (of
-  // both operands), v_rcp_f32, one Newton step of the reciprocal, the
-  // quotient and two residual corrections (the last through v_div_fmas),
-  // then v_div_fixup.  Where the operands need no scaling and the quotient
-  // no fixing (finite, |scale| in [2^-60, 2^60], |quotient| < 1024) the
-  // scalings are identities and v_div_fmas is a plain fma, so the same
-  // sequence without them gives the same bits; its reciprocal step depends
-  // on the scale only and is done once for the lane's elements.  Elsewhere
-  // (never for weights of ordinary magnitude) the division itself runs.
-  // A quotient below 1024 in magnitude but far smaller than the scale
-  // (|d| << |scale|) could still meet a scaled division; its code is 0
-  // either way (rint of a value far below 0.5).
-  const float r0 = __builtin_amdgcn_rcpf(scale);
-  const float r1 = fmaf(fmaf(-scale, r0, 1.0f), r0, r0);
-  const bool ordinary = fabsf(scale) >= 0x1p-60f && fabsf(scale) <= 0x1p60f;
-  bool any_other = !ordinary;  // one test for the lane's elements, one branch
+  recip(scale, r1, r2);
+  // false for an infinite or NaN edge too (a finite edge bounds the group)
+  const bool ordinary = fabsf(edge) <= 0x1p60f && (__float_as_uint(scale) & 0x7FFFFFu) != 0x7FFFFFu;
+  // The quotient lies in [0, n_bins + 1] (bias is the group's edge and scale
+  // of the sign that makes it positive; with bias 0 it rounds to 0); a NaN
+  // element clamps to 0.  Adding 2^23 rounds it to the nearest integer, ties
+  // to even, into the low mantissa bits; the words collect those bits, the
+  // exponent bits that the shifts leave behind are a constant.
 #pragma unroll
-  for (int i = 0; i < EPL; i++) {
-    const float d = v[i] - bias;
-    const float q0 = d * r1;
-    const float q1 = fmaf(fmaf(-scale, q0, d), r1, q0);
-    const float q2 = fmaf(fmaf(-scale, q1, d), r1, q1);
-    any_other |= !(fabsf(q0) < 1024.f);
-    codes[i] = static_cast<uint32_t>(fminf(fmaxf(__builtin_rintf(q2), 0.f), n_bins));
-  }
-  if (any_other) {
+  for (int w = 0; w < EPL / CPW; w++) {
+    uint32_t acc = 0;
 #pragma unroll
-    for (int i = 0; i < EPL; i++) {
-      const float d = v[i] - bias;
-      if (!(ordinary && fabsf(d * r1) < 1024.f))
-        codes[i] = static_cast<uint32_t>(fminf(fmaxf(__builtin_rintf(d / scale), 0.f), n_bins));
+    for (int i = CPW - 1; i >= 0; i--) {
+      const float d = v[w * CPW + i] - bias;
+      const float q = __builtin_amdgcn_fmed3f(fmaf(d, r1, d * r2), 0.f, n_bins);
+      acc = (acc << BITS) + __float_as_uint(q + 0x1p23f);
     }
+    words[w] = acc - (BITS == 4 ? 0xFB000000u : 0x4B000000u);  // sum of 0x4B000000 << BITS i
   }
-}
-
-// Pack 16 codes LSB-first: two words (Q4) or four (Q8) at 16-code index
-// `lane` (8-byte stores).
-template <int BITS>
-__device__ __forceinline__ void store_codes16(uint32_t* wq, int64_t lane, const uint32_t (&codes)[16]) {
-  uint32_t w[BITS / 2];
+  if (!ordinary) {  // the whole group takes it: the divisions themselves
+    scale = fmaxf((w_max - w_min) / n_bins, eps);
+    scale = mask ? scale : -scale;
+    const float qe = __builtin_rintf(edge / scale);
+    bias = 0.f;
+    if (qe != 0.f) {
+      scale = edge / qe;
+      bias = edge;
+    }
 #pragma unroll
-  for (int j = 0; j < BITS / 2; j++) {
-    w[j] = 0;
+    for (int w = 0; w < EPL / CPW; w++) {
+      words[w] = 0;
 #pragma unroll
-    for (int i = 0; i < 32 / BITS; i++) w[j] |= codes[j * (32 / BITS) + i] << (BITS * i);
-  }
-#pragma unroll
-  for (int j = 0; j < BITS / 4; j++) reinterpret_cast<uint2*>(wq)[lane * (BITS / 4) + j] = uint2{w[2 * j], w[2 * j + 1]};
-}
-
-// Pack 8 codes LSB-first: one word (Q4) or two (Q8) at lane index `lane`.
-template <int BITS>
-__device__ __forceinline__ void store_codes8(uint32_t* wq, int64_t lane, const uint32_t (&codes)[8]) {
-  if constexpr (BITS == 4) {
-    uint32_t word = 0;
-#pragma unroll
-    for (int i = 0; i < 8; i++) word |= codes[i] << (4 * i);
-    wq[lane] = word;
-  } else {
-    uint2 words;
-    words.x = codes[0] | (codes[1] << 8) | (codes[2] << 16) | (codes[3] << 24);
-    words.y = codes[4] | (codes[5] << 8) | (codes[6] << 16) | (codes[7] << 24);
-    reinterpret_cast<uint2*>(wq)[lane] = words;
+      for (int i = 0; i < CPW; i++) {
+        const float q = fminf(fmaxf(__builtin_rintf((v[w * CPW + i] - bias) / scale), 0.f), n_bins);
+        words[w] |= static_cast<uint32_t>(q) << (BITS * i);
+      }
+    }
   }
 }
 

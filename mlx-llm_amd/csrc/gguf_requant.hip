@@ -225,12 +225,14 @@ __global__ __launch_bounds__(kThreads) void gguf_requant_kernel(const uint8_t* _
 #pragma unroll
         for (int j = 0; j < kEpl; j++) v[j] = static_cast<float>(static_cast<__bf16>(v[j]));  // as_dtype(bf16): v_cvt_pk_bf16_f32, round to nearest even (a NaN payload cannot reach a code: max/min skip NaN and a NaN quotient clamps to 0)
       }
-      uint32_t codes[kEpl];
+      uint32_t words[kEpl * BITS / 32];
       float scale, bias;
-      quantize_group8<BITS, LPG, kEpl>(v, codes, scale, bias);  // every lane of the group takes part
+      quantize_group<BITS, LPG, kEpl>(v, words, scale, bias);  // every lane of the group takes part
       if (active) {
         const int64_t lane = static_cast<int64_t>(r) * lpr + l;
-        store_codes16<BITS>(wq, lane, codes);
+#pragma unroll
+        for (int j = 0; j < BITS / 4; j++)
+          reinterpret_cast<uint2*>(wq)[lane * (BITS / 4) + j] = make_uint2(words[2 * j], words[2 * j + 1]);
         if ((l & (LPG - 1)) == 0) {
           const int64_t g = lane / LPG;
           scales[g] = static_cast<uint16_t>(f32_to_bf16_bits(scale));

@@ -110,3 +110,44 @@ def test_codes_at_rounding_ties(torch_gpu, bits, factor):
     got = gpu_quantize(w, gs, bits, False)
     for r, g in zip(ref, got):
         assert np.array_equal(np.asarray(r).view(np.uint8), np.asarray(g).view(np.uint8))
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("bf16", [True, False])
+def test_groups_outside_the_ordinary_range(torch_gpu, bits, gs, bf16):
+    """Groups that leave the short quotient's range or sit on its edges: huge,
+    tiny and subnormal values, infinities, single NaN elements, a scale whose
+    mantissa is all ones with a quotient next to one half, and a row count
+    whose last workgroup is partial.  Codes bit-exact, scales and biases too
+    except for the payload of a NaN."""
+    rng = np.random.default_rng(5 + gs)
+    n_bins = (1 << bits) - 1
+    s1 = np.float32(float.fromhex("0x1.fffffep-7"))
+    half = (n_bins + 1) // 2
+    groups = [rng.normal(0, f, gs) for f in (1e-30, 1e-42, 1e-8, 3e-7, 2e18, 1e25, 1e37, 1e38)]
+    groups += [np.where(rng.random(gs) < 0.5, -3e38, 3e38), np.full(gs, -0.0)]
+    for bad in (np.inf, -np.inf, np.nan):
+        g = rng.normal(0, 0.02, gs)
+        g[gs // 2 + 3] = bad
+        groups.append(g)
+    edge = np.full(gs, float(half * s1))  # scale = edge / half: all mantissa bits set
+    edge[1] = float(-(half - 1) * s1)
+    edge[2::2] = float(half * s1) - 2.0**-7  # quotient 0.5 rounded from just above
+    groups += [edge, -edge]
+    rows = 37
+    w = rng.normal(0, 0.02, (rows, 4 * gs)).astype(np.float32)
+    flat = w.reshape(-1, gs)
+    for i, g in enumerate(groups):
+        with np.errstate(over="ignore", under="ignore"):
+            flat[5 * i] = g.astype(np.float32)
+    w = flat.reshape(rows, 4 * gs)
+    if bf16:
+        w = orc.f32_to_bf16(w).reshape(rows, 4 * gs)
+    ref = orc.affine_quantize(w, gs, bits, orc.BF16 if bf16 else orc.F32)
+    got = gpu_quantize(w, gs, bits, bf16)
+    assert np.array_equal(ref[0], got[0].view(np.uint32))
+    for r, g in zip(ref[1:], got[1:]):
+        r = orc.bf16_to_f32(np.asarray(r)) if bf16 else np.asarray(r)
+        g = orc.bf16_to_f32(np.asarray(g).view(np.uint16)) if bf16 else np.asarray(g)
+        assert np.array_equal(r.reshape(-1), g.reshape(-1), equal_nan=True)
