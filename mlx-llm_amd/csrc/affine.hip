@@ -81,49 +81,64 @@ __global__ __launch_bounds__(kThreads) void affine_quantize_kernel(const void* _
   }
 }
 
-// One lane per 8 elements: out = scale*q + bias in f32, then stored in DT.
-template <int DT, int BITS>
+// out = scale*q + bias in f32, then stored in DT.  Bound by HBM (4 bits or a
+// byte in, 2 or 4 bytes out per element).  A unit is one 16-byte store (8
+// bf16 or 4 f32 outputs) and its codes; a workgroup covers U runs of 256
+// units, every run's loads first.  Each wave instruction stores 1 KB
+// contiguously, so the outputs, which the kernel never reads back, go out
+// non-temporal and leave the caches to the codes: 14336 x 4096, bf16 Q4 / Q8
+// 31.0 / 35.0 -> 22.5 / 33.0 us, f32 Q4 / Q8 54.4 / 56.3 -> 39.2 / 52.9 (U =
+// 4: 22.8 / 32.5, 39.3 / 54.1; plain stores at U = 2: 30.7 / 34.2, 56.4 /
+// 53.9).
+template <int DT, int BITS, int U>
 __global__ __launch_bounds__(kThreads) void affine_dequantize_kernel(const uint32_t* __restrict__ wq,
                                                                       const void* __restrict__ scales,
                                                                       const void* __restrict__ biases,
-                                                                      int64_t n_lanes, int lanes_per_group,
-                                                                      void* __restrict__ out) {
-  const int64_t lane = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  if (lane >= n_lanes) return;
-  const int64_t g = lane / lanes_per_group;
-  const float s = load1<DT>(scales, g), b = load1<DT>(biases, g);
-  uint32_t q[8];
-  if constexpr (BITS == 4) {
-    uint32_t word = wq[lane];
+                                                                      int64_t n_units, int gshift,
+                                                                      u32x4* __restrict__ out) {
+  constexpr int E = DT == MLXQ_F32 ? 4 : 8;  // elements per unit
+  constexpr int CB = E * BITS / 8;           // code bytes per unit: 2, 4 or 8
+  const int64_t u0 = static_cast<int64_t>(blockIdx.x) * (kThreads * U) + threadIdx.x;
+  uint32_t q[U][2];
+  float s[U], b[U];
 #pragma unroll
-    for (int i = 0; i < 8; i++) q[i] = (word >> (4 * i)) & 0xFu;
-  } else {
-    uint2 words = reinterpret_cast<const uint2*>(wq)[lane];
+  for (int j = 0; j < U; j++) {
+    const int64_t u = min(u0 + j * kThreads, n_units - 1);  // clamped: no branch around the loads
+    if constexpr (CB == 2) {
+      q[j][0] = reinterpret_cast<const uint16_t*>(wq)[u];
+    } else if constexpr (CB == 4) {
+      q[j][0] = wq[u];
+    } else {
+      const uint2 t = reinterpret_cast<const uint2*>(wq)[u];
+      q[j][0] = t.x;
+      q[j][1] = t.y;
+    }
+    const int64_t g = u >> gshift;
+    s[j] = load1<DT>(scales, g);
+    b[j] = load1<DT>(biases, g);
+  }
+#pragma unroll
+  for (int j = 0; j < U; j++) {
+    const int64_t u = u0 + j * kThreads;
+    if (u >= n_units) return;
+    float r[E];
+#pragma unroll
+    for (int i = 0; i < E; i++) {
+      const uint32_t c = (q[j][i * BITS / 32] >> (i * BITS % 32)) & ((1u << BITS) - 1);
+      r[i] = s[j] * static_cast<float>(c) + b[j];
+    }
+    u32x4 o;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      q[i] = (words.x >> (8 * i)) & 0xFFu;
-      q[4 + i] = (words.y >> (8 * i)) & 0xFFu;
+      if constexpr (DT == MLXQ_F32) {
+        o[i] = __float_as_uint(r[i]);
+      } else {
+        // v_cvt_pk_bf16_f32: two values per instruction, round to nearest even
+        const bf16x2_t v = {static_cast<__bf16>(r[2 * i]), static_cast<__bf16>(r[2 * i + 1])};
+        o[i] = __builtin_bit_cast(uint32_t, v);
+      }
     }
-  }
-  float r[8];
-#pragma unroll
-  for (int i = 0; i < 8; i++) r[i] = s * static_cast<float>(q[i]) + b;
-  if constexpr (DT == MLXQ_F32) {
-    float4* o = reinterpret_cast<float4*>(static_cast<float*>(out) + lane * 8);
-    o[0] = make_float4(r[0], r[1], r[2], r[3]);
-    o[1] = make_float4(r[4], r[5], r[6], r[7]);
-  } else {
-    // v_cvt_pk_bf16_f32: two values per instruction, round to nearest even
-    auto pk = [](float lo, float hi) {
-      const bf16x2_t v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
-      return __builtin_bit_cast(uint32_t, v);
-    };
-    uint4 p;
-    p.x = pk(r[0], r[1]);
-    p.y = pk(r[2], r[3]);
-    p.z = pk(r[4], r[5]);
-    p.w = pk(r[6], r[7]);
-    reinterpret_cast<uint4*>(static_cast<uint16_t*>(out) + lane * 8)[0] = p;
+    __builtin_nontemporal_store(o, out + u);
   }
 }
 
@@ -151,6 +166,15 @@ void launch_quant(const void* w, int64_t n, int group_size, uint32_t* wq, void* 
     case 64: MLXQ_LAUNCH((affine_quantize_kernel<DT, BITS, 64 / EPL, EPL>), grid, dim3(kThreads), 0, st, w, lanes, wq, s, b); break;
     default: MLXQ_LAUNCH((affine_quantize_kernel<DT, BITS, 128 / EPL, EPL>), grid, dim3(kThreads), 0, st, w, lanes, wq, s, b); break;
   }
+}
+
+template <int DT, int BITS>
+void launch_dequant(const uint32_t* wq, const void* s, const void* b, int64_t n, int group_size, void* out,
+                    hipStream_t st) {
+  constexpr int U = 2, E = DT == MLXQ_F32 ? 4 : 8;
+  const int64_t units = n / E;
+  MLXQ_LAUNCH((affine_dequantize_kernel<DT, BITS, U>), dim3(ceil_div(units, kThreads * U)), dim3(kThreads), 0, st, wq, s,
+              b, units, __builtin_ctz(static_cast<unsigned>(group_size / E)), static_cast<u32x4*>(out));
 }
 
 }  // namespace
@@ -182,18 +206,16 @@ extern "C" int mlxq_dequantize(const uint32_t* wq, const void* scales, const voi
   clear_error();
   int rc = check_args(dtype, rows, cols, group_size, bits);
   if (rc) return rc;
-  const int64_t n_lanes = rows * cols / 8;
-  if (n_lanes == 0) return MLXQ_OK;
+  const int64_t n = rows * cols;
+  if (n == 0) return MLXQ_OK;
   if (!wq || !scales || !biases || !out) return fail(MLXQ_ERR_INVALID, "dequantize: null pointer");
   hipStream_t st = as_stream(stream);
-  dim3 grid(ceil_div(n_lanes, kThreads));
-  const int lpg = group_size / 8;
   if (dtype == MLXQ_F32) {
-    if (bits == 4) MLXQ_LAUNCH((affine_dequantize_kernel<MLXQ_F32, 4>), grid, dim3(kThreads), 0, st, wq, scales, biases, n_lanes, lpg, out);
-    else MLXQ_LAUNCH((affine_dequantize_kernel<MLXQ_F32, 8>), grid, dim3(kThreads), 0, st, wq, scales, biases, n_lanes, lpg, out);
+    if (bits == 4) launch_dequant<MLXQ_F32, 4>(wq, scales, biases, n, group_size, out, st);
+    else launch_dequant<MLXQ_F32, 8>(wq, scales, biases, n, group_size, out, st);
   } else {
-    if (bits == 4) MLXQ_LAUNCH((affine_dequantize_kernel<MLXQ_BF16, 4>), grid, dim3(kThreads), 0, st, wq, scales, biases, n_lanes, lpg, out);
-    else MLXQ_LAUNCH((affine_dequantize_kernel<MLXQ_BF16, 8>), grid, dim3(kThreads), 0, st, wq, scales, biases, n_lanes, lpg, out);
+    if (bits == 4) launch_dequant<MLXQ_BF16, 4>(wq, scales, biases, n, group_size, out, st);
+    else launch_dequant<MLXQ_BF16, 8>(wq, scales, biases, n, group_size, out, st);
   }
   return check_launch("dequantize");
 }

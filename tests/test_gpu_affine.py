@@ -151,3 +151,21 @@ def test_groups_outside_the_ordinary_range(torch_gpu, bits, gs, bf16):
         r = orc.bf16_to_f32(np.asarray(r)) if bf16 else np.asarray(r)
         g = orc.bf16_to_f32(np.asarray(g).view(np.uint16)) if bf16 else np.asarray(g)
         assert np.array_equal(r.reshape(-1), g.reshape(-1), equal_nan=True)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("rows,cols", [(1, 128), (3, 384), (33, 640)])
+def test_dequantize_partial_workgroups(torch_gpu, bits, gs, bf16, rows, cols):
+    import torch
+
+    w = bf16_weights(77 + bits, rows, cols)
+    if not bf16:
+        w = orc.normal(78 + bits, rows * cols, 0, 0.02).reshape(rows, cols)
+    dt = orc.BF16 if bf16 else orc.F32
+    wq, s, b = orc.affine_quantize(w, gs, bits, dt)
+    ref = orc.affine_dequantize(wq, s, b, gs, bits, dt)
+    got = mlxq.dequantize(dev(wq), dev(s, bf16=bf16), dev(b, bf16=bf16), gs, bits)
+    torch.cuda.synchronize()
+    assert np.array_equal(host(got).view(np.uint8), np.asarray(ref).view(np.uint8))
