@@ -51,12 +51,14 @@ __device__ __forceinline__ void quantize_group(const float (&v)[EPL], uint32_t (
     w_min = fminf(w_min, v[i]);
   }
   // All-reduce within the LPG lanes of this group (groups never straddle a
-  // 16-lane row: LPG is 2 .. 16 and the lane index is group-aligned) with
+  // 16-lane row: LPG is 1 .. 16 and the lane index is group-aligned) with
   // DPP moves: quad swaps, then the other quad of 8 (lane i <-> 7 - i), then
   // the other 8 of 16 (i <-> 15 - i).  Exact for max/min in any order.
-  static_assert(LPG == 2 || LPG == 4 || LPG == 8 || LPG == 16, "lanes per group");
-  w_max = fmaxf(w_max, dpp_all<kDppQuadXor1>(w_max));
-  w_min = fminf(w_min, dpp_all<kDppQuadXor1>(w_min));
+  static_assert(LPG == 1 || LPG == 2 || LPG == 4 || LPG == 8 || LPG == 16, "lanes per group");
+  if constexpr (LPG >= 2) {
+    w_max = fmaxf(w_max, dpp_all<kDppQuadXor1>(w_max));
+    w_min = fminf(w_min, dpp_all<kDppQuadXor1>(w_min));
+  }
   if constexpr (LPG >= 4) {
     w_max = fmaxf(w_max, dpp_all<kDppQuadXor2>(w_max));
     w_min = fminf(w_min, dpp_all<kDppQuadXor2>(w_min));

@@ -16,7 +16,6 @@
 #include <string>
 
 #include "common.hpp"
-#define MLXQ_IQ4NL_IN_REGISTERS 1  // IQ4 codebook lookups by v_perm (this kernel is memory-bound)
 #include "gguf_decode.hpp"
 
 namespace mlxq {
@@ -34,24 +33,14 @@ __device__ __forceinline__ uint32_t pack_bf16_rne(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
-template <bool BF16OUT>
-__device__ __forceinline__ void store_vec(void* out, int64_t e, const float (&v)[kVec]) {
-  if constexpr (BF16OUT) {
-    // v_cvt_pk_bf16_f32: round to nearest even, two values per instruction
-    // (the same bits as f32_to_bf16_bits except NaN payloads)
-    uint4 p;
-    p.x = pack_bf16_rne(v[0], v[1]);
-    p.y = pack_bf16_rne(v[2], v[3]);
-    p.z = pack_bf16_rne(v[4], v[5]);
-    p.w = pack_bf16_rne(v[6], v[7]);
-    // written once and not read back by this kernel: non-temporal (each
-    // wave instruction covers 1 KB contiguously)
-    __builtin_nontemporal_store(u32x4{p.x, p.y, p.z, p.w}, reinterpret_cast<u32x4*>(static_cast<uint16_t*>(out) + e));
-  } else {
-    float4* o = reinterpret_cast<float4*>(static_cast<float*>(out) + e);
-    o[0] = make_float4(v[0], v[1], v[2], v[3]);
-    o[1] = make_float4(v[4], v[5], v[6], v[7]);
-  }
+__device__ __forceinline__ void store_bf16x8(void* out, int64_t e, const float (&v)[kVec]) {
+  // v_cvt_pk_bf16_f32: round to nearest even, two values per instruction
+  // (the same bits as f32_to_bf16_bits except NaN payloads).  Written once
+  // and not read back by this kernel: non-temporal (each wave instruction
+  // covers 1 KB contiguously)
+  __builtin_nontemporal_store(u32x4{pack_bf16_rne(v[0], v[1]), pack_bf16_rne(v[2], v[3]), pack_bf16_rne(v[4], v[5]),
+                                    pack_bf16_rne(v[6], v[7])},
+                              reinterpret_cast<u32x4*>(static_cast<uint16_t*>(out) + e));
 }
 
 // One workgroup per kCpw chunks of kChunkElems elements (each a whole number
@@ -67,40 +56,6 @@ constexpr int kCpw = 4;
 // fill 1 KB from `l`)
 __device__ __forceinline__ void lds_dma16(const uint8_t* g, uint8_t* l) {
   __builtin_amdgcn_global_load_lds(g, l, 16, 0, 0);
-}
-
-// f32 output in two 1 KB halves per store pass (measured, µs for a 14336 x
-// 4096 tensor: Q4_0 53.3 -> 47.6, Q8_0 61 -> 51.7, Q6_K 56.5 -> 49.6,
-// IQ4_NL 52 -> 47.4, IQ4_XS 52 -> 48; Q4_K with its 4-element run decoder
-// 58 -> 48); the other formats keep 8 consecutive elements per thread
-template <int TAG>
-constexpr bool f32_halves() {
-  return TAG == 2 || TAG == 8 || TAG == 12 || TAG == 14 || TAG == 20 || TAG == 23;
-}
-
-// Q4_K elements j .. j + N - 1 (one sub-block, one nibble half) with
-// decode<12>'s arithmetic in its order: the sub-block's scale and min and
-// the block's d, dmin derived once for the run
-// (N = 4 or 8: j a multiple of N; the run's bytes are N-byte aligned)
-template <int N>
-__device__ __forceinline__ void q4k_run(const uint8_t* b, int j, float* v) {
-  const int c = j >> 6, hi = (j >> 5) & 1, l = j & 31;
-  uint32_t sc, m;
-  scale_min_k4(2 * c + hi, b + 4, sc, m);
-  const float d = rd_f16(b, 0), dmin = rd_f16(b, 2);
-  const float d1 = d * static_cast<float>(sc);
-  const float m1 = dmin * static_cast<float>(m);
-  uint32_t w[N / 4];
-  if constexpr (N == 8) {
-    const uint2 q = *reinterpret_cast<const uint2*>(b + 16 + 32 * c + l);
-    w[0] = q.x;
-    w[1] = q.y;
-  } else {
-    w[0] = *reinterpret_cast<const uint32_t*>(b + 16 + 32 * c + l);
-  }
-  const int sh = 4 * hi;
-#pragma unroll
-  for (int i = 0; i < N; i++) v[i] = d1 * static_cast<float>((w[i >> 2] >> (8 * (i & 3) + sh)) & 0xFu) - m1;
 }
 
 template <int TAG, bool BF16OUT, bool ALIGNED16>
@@ -140,24 +95,25 @@ __global__ __launch_bounds__(kThreads) void gguf_dequant_kernel(const uint8_t* _
 
 #pragma unroll
   for (int c = 0; c < kCpw; c++) {
-    if constexpr (!BF16OUT && f32_halves<TAG>()) {
+    if constexpr (!BF16OUT) {
       // f32 out: elements tid * 4 .. +3 and 1024 + tid * 4 .. +3 of the
       // chunk, so that each of the two 16-byte store instructions covers 1
       // KB contiguously and can go out non-temporal (with 32 bytes per lane
       // each instruction would cover every line half, and non-temporal
-      // half-line stores measured nearly twice as slow)
+      // half-line stores measured nearly twice as slow).  14336 x 4096 (us,
+      // 8 consecutive elements per thread and a per-element decode -> here):
+      // Q2_K 48.1 -> 42.4, Q3_K 63.3 -> 42.7, Q5_K 55.9 -> 41.1, Q5_0 55.0
+      // -> 52.1; Q4_0 53.3 -> 42, Q8_0 61 -> 53, Q4_K 58 -> 40.5
       const int e0 = c * kChunkElems + tid * 4;
       if (e0 >= nb * E) return;  // the second half lies beyond the first
       float v[kVec];
 #pragma unroll
       for (int h = 0; h < 2; h++) {
         const int e = e0 + h * (kThreads * 4);
-        if constexpr (TAG == 12) {
-          q4k_run<4>(lds + (e / E) * B, e % E, v + 4 * h);
-        } else {
+        float t[4];
+        decode_run<TAG, 4>(lds + (e / E) * B, e % E, t);
 #pragma unroll
-          for (int i = 0; i < 4; i++) v[4 * h + i] = decode<TAG>(lds + ((e + i) / E) * B, (e + i) % E);
-        }
+        for (int i = 0; i < 4; i++) v[4 * h + i] = t[i];
       }
       f32x4* o = reinterpret_cast<f32x4*>(static_cast<float*>(out) + static_cast<int64_t>(blockIdx.x) * kCpw * kChunkElems + e0);
       __builtin_nontemporal_store(f32x4{v[0], v[1], v[2], v[3]}, o);
@@ -166,16 +122,8 @@ __global__ __launch_bounds__(kThreads) void gguf_dequant_kernel(const uint8_t* _
       const int e0 = c * kChunkElems + tid * kVec;  // element within the workgroup
       if (e0 >= nb * E) return;
       float v[kVec];
-      if constexpr (TAG == 12) {
-        q4k_run<8>(lds + (e0 / E) * B, e0 % E, v);
-      } else {
-#pragma unroll
-        for (int i = 0; i < kVec; i++) {
-          const int e = e0 + i;
-          v[i] = decode<TAG>(lds + (e / E) * B, e % E);
-        }
-      }
-      store_vec<BF16OUT>(out, static_cast<int64_t>(blockIdx.x) * kCpw * kChunkElems + e0, v);
+      decode_run<TAG, kVec>(lds + (e0 / E) * B, e0 % E, v);
+      store_bf16x8(out, static_cast<int64_t>(blockIdx.x) * kCpw * kChunkElems + e0, v);
     }
   }
 }
@@ -188,10 +136,12 @@ __global__ __launch_bounds__(kThreads) void gguf_float_kernel(const uint8_t* __r
   if (e >= n) return;
   float v;
   if (TAG == 0) {
-    v = bits_to_f32(rd_u32(data + 4 * e));
+    uint32_t w;
+    __builtin_memcpy(&w, data + 4 * e, 4);
+    v = bits_to_f32(w);
   } else {
     uint32_t h = static_cast<uint32_t>(data[2 * e]) | (static_cast<uint32_t>(data[2 * e + 1]) << 8);
-    v = TAG == 1 ? f16_bits_to_f32(h) : bf16_bits_to_f32(h);
+    v = TAG == 1 ? f16_to_f32(h) : bf16_bits_to_f32(h);
   }
   if constexpr (BF16OUT) static_cast<uint16_t*>(out)[e] = static_cast<uint16_t>(f32_to_bf16_bits(v));
   else static_cast<float*>(out)[e] = v;

@@ -1,12 +1,17 @@
 // GGUF block decoding shared by the dequantizer (gguf.hip) and the fused
 // dequantize + requantize converter (gguf_requant.hip).
 //
-// Reference: the per-type block decoders of src/gguf/dequant.rs (:228-719),
-// solved for one element: decode<TAG>(block, j) is element j of a block, with
-// exactly the IEEE f32 operations, operand order and roundings the reference
-// uses for it.  Every file that includes this header is compiled with
-// -ffp-contract=off so no mul+add/sub is fused; f16 scales are decoded with
-// integer bit operations.
+// Reference: the per-type block decoders of src/gguf/dequant.rs (:228-719).
+// decode_run<TAG, N>(block, j, v) is elements j .. j + N - 1 of a block (N =
+// 4, 8, 16 or 32, j a multiple of N), with exactly the IEEE f32 operations,
+// operand order and roundings the reference uses for each.  Every file that
+// includes this header is compiled with -ffp-contract=off so no mul+add/sub
+// is fused.
+//
+// A run shares what its elements have in common: the f16 block scales (one
+// v_cvt_f32_f16 each, exact for every encoding), the sub-block scale, the
+// nibble half; codes are masked four at a time in their words and converted
+// with one instruction each.  Blocks are read from LDS at 2-byte alignment.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -17,42 +22,65 @@
 namespace mlxq {
 namespace {  // internal linkage: each including file has its own copy
 
+__device__ __forceinline__ float f16_to_f32(uint32_t h) {
+  return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(h)));
+}
+// 2-byte aligned reads (every block size and field offset used here is even)
+__device__ __forceinline__ uint32_t rd_u16(const uint8_t* b) { return *reinterpret_cast<const uint16_t*>(b); }
+__device__ __forceinline__ float rd_f16(const uint8_t* b, int i) { return f16_to_f32(rd_u16(b + i)); }
+__device__ __forceinline__ uint32_t rd_u32(const uint8_t* b) { return rd_u16(b) | (rd_u16(b + 2) << 16); }
+// N bytes at alignment A as words
+template <int N, int A>
+__device__ __forceinline__ void rd_words(const uint8_t* b, uint32_t (&w)[N / 4]) {
+  __builtin_memcpy(w, __builtin_assume_aligned(b, A), N);
+}
+
+// float of unsigned byte k of a word (v_cvt_f32_ubyte)
+__device__ __forceinline__ float ubyte(uint32_t w, int k) { return static_cast<float>((w >> (8 * k)) & 0xFFu); }
+// float of signed byte k
+__device__ __forceinline__ float sbyte(uint32_t w, int k) {
+  return static_cast<float>(static_cast<int8_t>((w >> (8 * k)) & 0xFFu));
+}
+
+// f(i, w) for the N/4 words w of a run whose four codes sit in the nibbles of
+// four bytes: 16 bytes at p hold elements 0-15 in the low nibbles and 16-31
+// in the high ones (Q4_0 and its kin)
+template <int N, int A, typename F>
+__device__ __forceinline__ void nibbles16(const uint8_t* p, int j, F&& f) {
+  if constexpr (N == 32) {
+    uint32_t w[4];
+    rd_words<16, A>(p, w);
+#pragma unroll
+    for (int i = 0; i < 8; i++) f(i, (i < 4 ? w[i & 3] : w[i & 3] >> 4) & 0x0F0F0F0Fu);
+  } else {
+    uint32_t w[N / 4];
+    rd_words<N, (A < N ? A : N)>(p + (j & 15), w);
+    const int sh = (j >> 2) & 4;
+#pragma unroll
+    for (int i = 0; i < N / 4; i++) f(i, (w[i] >> sh) & 0x0F0F0F0Fu);
+  }
+}
+
+// bits 0-3 of x as the low bits of four bytes
+__device__ __forceinline__ uint32_t spread4(uint32_t x) { return __umul24(x & 0xFu, 0x204081u) & 0x01010101u; }
+
+// IQ4_NL codebook, four lookups at once: v_perm picks byte q & 7 of each
+// 8-byte half of the table, and a byte mask of the codes' bit 3 (selectors
+// 8-11 of v_perm replicate a sign bit) selects between the halves.
 constexpr int8_t kIq4nl[16] = {-127, -104, -83, -65, -49, -35, -22, -10,
                                1,    13,   25,  38,  53,  69,  89,  113};
-// The codebook as four little-endian dwords of bytes, so a lookup is a
-// v_perm byte select in registers instead of a per-lane memory load.
 constexpr uint32_t iq4nl_word(int w) {
   return static_cast<uint32_t>(static_cast<uint8_t>(kIq4nl[4 * w])) |
          (static_cast<uint32_t>(static_cast<uint8_t>(kIq4nl[4 * w + 1])) << 8) |
          (static_cast<uint32_t>(static_cast<uint8_t>(kIq4nl[4 * w + 2])) << 16) |
          (static_cast<uint32_t>(static_cast<uint8_t>(kIq4nl[4 * w + 3])) << 24);
 }
-// kIq4nl[q] for q in 0..15.  Two forms, chosen per including file by what
-// measured faster there: the memory-bound dequantizer defines
-// MLXQ_IQ4NL_IN_REGISTERS (v_perm picks byte q & 7 of the 8-byte half
-// selected by q & 8; selector values 0-3 address the second operand: 51 ->
-// 44 us for a 14336x4096 IQ4_NL tensor), the VALU-bound converter keeps the
-// table load (56 vs 61 us with the v_perm form).
-#ifdef MLXQ_IQ4NL_IN_REGISTERS
-__device__ __forceinline__ int iq4nl_value(uint32_t q) {
-  const uint32_t sel = q & 7u;
+__device__ __forceinline__ uint32_t iq4nl_values(uint32_t q) {  // four codes in bytes -> four signed bytes
+  const uint32_t sel = q & 0x07070707u, y = q << 4;
   const uint32_t lo = __builtin_amdgcn_perm(iq4nl_word(1), iq4nl_word(0), sel);
   const uint32_t hi = __builtin_amdgcn_perm(iq4nl_word(3), iq4nl_word(2), sel);
-  return static_cast<int8_t>((q & 8u) ? hi : lo);
-}
-#else
-__constant__ int8_t kIq4nlDev[16] = {kIq4nl[0],  kIq4nl[1],  kIq4nl[2],  kIq4nl[3],  kIq4nl[4],  kIq4nl[5],
-                                     kIq4nl[6],  kIq4nl[7],  kIq4nl[8],  kIq4nl[9],  kIq4nl[10], kIq4nl[11],
-                                     kIq4nl[12], kIq4nl[13], kIq4nl[14], kIq4nl[15]};
-__device__ __forceinline__ int iq4nl_value(uint32_t q) { return kIq4nlDev[q]; }
-#endif
-
-__device__ __forceinline__ float rd_f16(const uint8_t* b, int i) {
-  return f16_bits_to_f32(static_cast<uint32_t>(b[i]) | (static_cast<uint32_t>(b[i + 1]) << 8));
-}
-__device__ __forceinline__ uint32_t rd_u32(const uint8_t* b) {
-  return static_cast<uint32_t>(b[0]) | (static_cast<uint32_t>(b[1]) << 8) |
-         (static_cast<uint32_t>(b[2]) << 16) | (static_cast<uint32_t>(b[3]) << 24);
+  const uint32_t mask = __builtin_amdgcn_perm(y << 8, y, 0x090B080Au);
+  return (hi & mask) | (lo & ~mask);
 }
 
 // get_scale_min_k4 (dequant.rs:375-383).  Branch-free (j differs between
@@ -62,158 +90,15 @@ __device__ __forceinline__ uint32_t rd_u32(const uint8_t* b) {
 __device__ __forceinline__ void scale_min_k4(int j, const uint8_t* q, uint32_t& d, uint32_t& m) {
   const int j3 = j & 3;
   const uint32_t a = q[j3], b = q[j3 + 4], c = q[j3 + 8];
-  const bool low = j < 4;
-  d = low ? (a & 63u) : ((c & 0x0Fu) | ((a >> 6) << 4));
-  m = low ? (b & 63u) : ((c >> 4) | ((b >> 6) << 4));
+  const uint32_t hd = (c & 0x0Fu) | ((a >> 6) << 4), hm = (c >> 4) | ((b >> 6) << 4);
+  const uint32_t low = j < 4 ? 0xFFu : 0u;
+  d = (a & 63u & low) | (hd & ~low);
+  m = (b & 63u & low) | (hm & ~low);
 }
 
-// One element j of a block at b (LDS).  Tag is a template constant.
+// One element j of a block at b (LDS): the IQ grid types.
 template <int TAG>
 __device__ __forceinline__ float decode(const uint8_t* b, int j);
-
-// Q4_0 (dequant.rs:228-237): y[j]=(lo-8)*d, y[j+16]=(hi-8)*d
-template <>
-__device__ __forceinline__ float decode<2>(const uint8_t* b, int j) {
-  float d = rd_f16(b, 0);
-  uint32_t byte = b[2 + (j & 15)];
-  int q = static_cast<int>(j < 16 ? (byte & 0xFu) : (byte >> 4)) - 8;
-  return static_cast<float>(q) * d;
-}
-// Q4_1 (dequant.rs:239-247): q*d + m
-template <>
-__device__ __forceinline__ float decode<3>(const uint8_t* b, int j) {
-  float d = rd_f16(b, 0), m = rd_f16(b, 2);
-  uint32_t byte = b[4 + (j & 15)];
-  uint32_t q = j < 16 ? (byte & 0xFu) : (byte >> 4);
-  return static_cast<float>(q) * d + m;
-}
-// Q5_0 (dequant.rs:249-261)
-template <>
-__device__ __forceinline__ float decode<6>(const uint8_t* b, int j) {
-  float d = rd_f16(b, 0);
-  uint32_t qh = rd_u32(b + 2);
-  int jj = j & 15;
-  uint32_t byte = b[6 + jj];
-  uint32_t x;
-  if (j < 16) x = (byte & 0xFu) | (((qh >> jj) << 4) & 0x10u);
-  else x = (byte >> 4) | ((qh >> (jj + 12)) & 0x10u);
-  return static_cast<float>(static_cast<int>(x) - 16) * d;
-}
-// Q5_1 (dequant.rs:263-276)
-template <>
-__device__ __forceinline__ float decode<7>(const uint8_t* b, int j) {
-  float d = rd_f16(b, 0), m = rd_f16(b, 2);
-  uint32_t qh = rd_u32(b + 4);
-  int jj = j & 15;
-  uint32_t byte = b[8 + jj];
-  uint32_t x;
-  if (j < 16) x = (byte & 0xFu) | (((qh >> jj) << 4) & 0x10u);
-  else x = (byte >> 4) | ((qh >> (jj + 12)) & 0x10u);
-  return static_cast<float>(x) * d + m;
-}
-// Q8_0 (dequant.rs:278-284)
-template <>
-__device__ __forceinline__ float decode<8>(const uint8_t* b, int j) {
-  float d = rd_f16(b, 0);
-  return static_cast<float>(static_cast<int8_t>(b[2 + j])) * d;
-}
-// Q2_K (dequant.rs:288-318): element j -> half h (128), shift round r (32),
-// 16-lane half l2/16 selecting scales[8h + 2r + l2/16].
-template <>
-__device__ __forceinline__ float decode<10>(const uint8_t* b, int j) {
-  int h = j >> 7, r = (j >> 5) & 3, l2 = j & 31;
-  uint32_t sc = b[8 * h + 2 * r + (l2 >> 4)];
-  float d = rd_f16(b, 80), dmin = rd_f16(b, 82);
-  float dl = d * static_cast<float>(sc & 0xFu);
-  float ml = dmin * static_cast<float>(sc >> 4);
-  uint32_t qb = b[16 + 32 * h + l2];
-  return dl * static_cast<float>((qb >> (2 * r)) & 3u) - ml;
-}
-// Q3_K (dequant.rs:320-371)
-template <>
-__device__ __forceinline__ float decode<11>(const uint8_t* b, int j) {
-  const uint32_t K1 = 0x03030303u, K2 = 0x0f0f0f0fu;
-  int h = j >> 7, r = (j >> 5) & 3, l2 = j & 31;
-  int is = 8 * h + 2 * r + (l2 >> 4);
-  uint32_t a0 = rd_u32(b + 96), a1 = rd_u32(b + 100), tmp = rd_u32(b + 104);
-  uint32_t aux;
-  switch (is >> 2) {
-    case 0: aux = (a0 & K2) | ((tmp & K1) << 4); break;
-    case 1: aux = (a1 & K2) | (((tmp >> 2) & K1) << 4); break;
-    case 2: aux = ((a0 >> 4) & K2) | (((tmp >> 4) & K1) << 4); break;
-    default: aux = ((a1 >> 4) & K2) | (((tmp >> 6) & K1) << 4); break;
-  }
-  int sc = static_cast<int8_t>((aux >> (8 * (is & 3))) & 0xFFu);
-  float d_all = rd_f16(b, 108);
-  float dl = d_all * static_cast<float>(sc - 32);
-  uint32_t m = 1u << (4 * h + r);
-  int hbit = (b[l2] & m) ? 0 : 4;
-  uint32_t qb = b[32 + 32 * h + l2];
-  return dl * static_cast<float>(static_cast<int>((qb >> (2 * r)) & 3u) - hbit);
-}
-// Q4_K (dequant.rs:385-410)
-template <>
-__device__ __forceinline__ float decode<12>(const uint8_t* b, int j) {
-  int c = j >> 6, hi = (j >> 5) & 1, l = j & 31;
-  uint32_t sc, m;
-  scale_min_k4(2 * c + hi, b + 4, sc, m);
-  float d = rd_f16(b, 0), dmin = rd_f16(b, 2);
-  float d1 = d * static_cast<float>(sc);
-  float m1 = dmin * static_cast<float>(m);
-  uint32_t qb = b[16 + 32 * c + l];
-  uint32_t q = hi ? (qb >> 4) : (qb & 0xFu);
-  return d1 * static_cast<float>(q) - m1;
-}
-// Q5_K (dequant.rs:412-444)
-template <>
-__device__ __forceinline__ float decode<13>(const uint8_t* b, int j) {
-  int c = j >> 6, hi = (j >> 5) & 1, l = j & 31;
-  uint32_t sc, m;
-  scale_min_k4(2 * c + hi, b + 4, sc, m);
-  float d = rd_f16(b, 0), dmin = rd_f16(b, 2);
-  float d1 = d * static_cast<float>(sc);
-  float m1 = dmin * static_cast<float>(m);
-  uint32_t u = (hi ? 2u : 1u) << (2 * c);
-  int hib = (b[16 + l] & u) ? 16 : 0;
-  uint32_t qb = b[48 + 32 * c + l];
-  int q = static_cast<int>(hi ? (qb >> 4) : (qb & 0xFu)) + hib;
-  return d1 * static_cast<float>(q) - m1;
-}
-// Q6_K (dequant.rs:446-468): (d * scale) * q, left to right
-template <>
-__device__ __forceinline__ float decode<14>(const uint8_t* b, int j) {
-  int idx = j >> 7, t = (j >> 5) & 3, l = j & 31;
-  const uint8_t* qlp = b + 64 * idx;
-  const uint8_t* qhp = b + 128 + 32 * idx;
-  // branch-free: byte l or l + 32 of ql, low or high nibble
-  const uint32_t lo = (static_cast<uint32_t>(qlp[l + 32 * (t & 1)]) >> (4 * (t >> 1))) & 0xFu;
-  uint32_t hb = (qhp[l] >> (2 * t)) & 3u;
-  int q = static_cast<int>(static_cast<int8_t>(lo | (hb << 4))) - 32;
-  int sc = static_cast<int8_t>(b[192 + 8 * idx + (l >> 4) + 2 * t]);
-  float d = rd_f16(b, 208);
-  return d * static_cast<float>(sc) * static_cast<float>(q);
-}
-// IQ4_NL (dequant.rs:472-479)
-template <>
-__device__ __forceinline__ float decode<20>(const uint8_t* b, int j) {
-  float d = rd_f16(b, 0);
-  uint32_t byte = b[2 + (j & 15)];
-  uint32_t q = j < 16 ? (byte & 0xFu) : (byte >> 4);
-  return d * static_cast<float>(iq4nl_value(q));
-}
-// IQ4_XS (dequant.rs:481-497)
-template <>
-__device__ __forceinline__ float decode<23>(const uint8_t* b, int j) {
-  int ib = j >> 5, jj = j & 31;
-  float d = rd_f16(b, 0);
-  uint32_t sh = static_cast<uint32_t>(b[2]) | (static_cast<uint32_t>(b[3]) << 8);
-  int ls = static_cast<int>((b[4 + (ib >> 1)] >> (4 * (ib & 1))) & 0xFu) |
-           static_cast<int>(((sh >> (2 * ib)) & 3u) << 4);
-  float dl = d * static_cast<float>(ls - 32);
-  uint32_t byte = b[8 + 16 * ib + (jj & 15)];
-  uint32_t q = jj < 16 ? (byte & 0xFu) : (byte >> 4);
-  return dl * static_cast<float>(iq4nl_value(q));
-}
 
 // ---- IQ grid types (dequant.rs:505-719).  Codebooks: the format's fixed
 // tables (iq_tables.h).  ksigns_iq2xs is computed: entry i is i with bit 7 =
@@ -315,7 +200,7 @@ __device__ __forceinline__ float decode<29>(const uint8_t* b, int j) {
 #pragma unroll
   for (int i = 0; i < 4; i++) sc[i] = static_cast<uint32_t>(b[48 + 2 * i]) | (static_cast<uint32_t>(b[49 + 2 * i]) << 8);
   const uint32_t bits = (sc[0] >> 12) | ((sc[1] >> 8) & 0x00F0u) | ((sc[2] >> 4) & 0x0F00u) | (sc[3] & 0xF000u);
-  const float d = f16_bits_to_f32(bits);
+  const float d = f16_to_f32(bits);
   const uint32_t w = sc[ib >> 1];
   const int shift = 6 * (ib & 1) + (l < 2 ? 0 : 3);
   const float dl = d * static_cast<float>(2 * static_cast<int>((w >> shift) & 7u) + 1);
@@ -324,6 +209,129 @@ __device__ __forceinline__ float decode<29>(const uint8_t* b, int j) {
   const float delta = (qh & ((l & 1) ? 0x80u : 0x08u)) ? -kIq1sDelta : kIq1sDelta;
   const int v = static_cast<int8_t>(grid_byte(kIq1s[idx], jj));
   return dl * (static_cast<float>(v) + delta);
+}
+
+template <int TAG, int N>
+__device__ __forceinline__ void decode_run(const uint8_t* b, int j, float (&v)[N]) {
+  static_assert(N == 4 || N == 8 || N == 16 || N == 32, "run length");
+  if constexpr (TAG == 2) {  // Q4_0 (dequant.rs:228-237): (q - 8) * d
+    const float d = rd_f16(b, 0);
+    nibbles16<N, 2>(b + 2, j, [&](int i, uint32_t w) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) v[4 * i + k] = (ubyte(w, k) - 8.f) * d;
+    });
+  } else if constexpr (TAG == 3) {  // Q4_1 (dequant.rs:239-247): q * d + m
+    const float d = rd_f16(b, 0), m = rd_f16(b, 2);
+    nibbles16<N, 4>(b + 4, j, [&](int i, uint32_t w) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) v[4 * i + k] = ubyte(w, k) * d + m;
+    });
+  } else if constexpr (TAG == 6) {  // Q5_0 (dequant.rs:249-261): (q - 16) * d, fifth bits in qh
+    const float d = rd_f16(b, 0);
+    const uint32_t qh = rd_u32(b + 2) >> (j & 31);
+    nibbles16<N, 2>(b + 6, j, [&](int i, uint32_t w) {
+      const uint32_t x = w | (spread4(qh >> (4 * i)) << 4);
+#pragma unroll
+      for (int k = 0; k < 4; k++) v[4 * i + k] = (ubyte(x, k) - 16.f) * d;
+    });
+  } else if constexpr (TAG == 7) {  // Q5_1 (dequant.rs:263-276): q * d + m
+    const float d = rd_f16(b, 0), m = rd_f16(b, 2);
+    const uint32_t qh = rd_u32(b + 4) >> (j & 31);
+    nibbles16<N, 8>(b + 8, j, [&](int i, uint32_t w) {
+      const uint32_t x = w | (spread4(qh >> (4 * i)) << 4);
+#pragma unroll
+      for (int k = 0; k < 4; k++) v[4 * i + k] = ubyte(x, k) * d + m;
+    });
+  } else if constexpr (TAG == 8) {  // Q8_0 (dequant.rs:278-284)
+    const float d = rd_f16(b, 0);
+    uint32_t w[N / 4];
+    rd_words<N, 2>(b + 2 + j, w);
+#pragma unroll
+    for (int e = 0; e < N; e++) v[e] = sbyte(w[e >> 2], e & 3) * d;
+  } else if constexpr (TAG == 10 || TAG == 11 || TAG == 14) {
+    // 16 elements a scale: half h (128 elements), 32-run r, byte l of the run
+    constexpr int S = N < 16 ? N : 16;
+    const int h = j >> 7, r = (j >> 5) & 3;
+    const float d = rd_f16(b, TAG == 10 ? 80 : TAG == 11 ? 108 : 208);
+    const float dmin = TAG == 10 ? rd_f16(b, 82) : 0.f;
+#pragma unroll
+    for (int g = 0; g < N / S; g++) {
+      const int l = (j & 31) + g * S, is = 8 * h + 2 * r + (l >> 4);
+      float (&o)[N] = v;
+      uint32_t w[S / 4];
+      if constexpr (TAG == 10) {  // Q2_K (dequant.rs:288-318): dl * q - ml
+        const uint32_t sc = b[is];
+        const float dl = d * static_cast<float>(sc & 0xFu), ml = dmin * static_cast<float>(sc >> 4);
+        rd_words<S, 4>(b + 16 + 32 * h + l, w);
+#pragma unroll
+        for (int i = 0; i < S / 4; i++) {
+          const uint32_t x = (w[i] >> (2 * r)) & 0x03030303u;
+#pragma unroll
+          for (int k = 0; k < 4; k++) o[g * S + 4 * i + k] = dl * ubyte(x, k) - ml;
+        }
+      } else if constexpr (TAG == 11) {  // Q3_K (dequant.rs:320-371): dl * (2-bit code - 4 where the mask bit is clear)
+        const int sc = static_cast<int>(((b[96 + (is & 7)] >> (4 * (is >> 3))) & 0xFu) |
+                                        (((b[104 + (is & 3)] >> (2 * (is >> 2))) & 3u) << 4));
+        const float dl = d * static_cast<float>(sc - 32);
+        uint32_t m[S / 4];
+        rd_words<S, 2>(b + 32 + 32 * h + l, w);
+        rd_words<S, 2>(b + l, m);
+#pragma unroll
+        for (int i = 0; i < S / 4; i++) {
+          const uint32_t x = ((w[i] >> (2 * r)) & 0x03030303u) | (((m[i] >> (4 * h + r)) & 0x01010101u) << 2);
+#pragma unroll
+          for (int k = 0; k < 4; k++) o[g * S + 4 * i + k] = dl * (ubyte(x, k) - 4.f);
+        }
+      } else {  // Q6_K (dequant.rs:446-468): (d * scale) * (q - 32)
+        const float ds = d * static_cast<float>(static_cast<int8_t>(b[192 + is]));
+        uint32_t u[S / 4];
+        rd_words<S, 2>(b + 64 * h + 32 * (r & 1) + l, w);
+        rd_words<S, 2>(b + 128 + 32 * h + l, u);
+#pragma unroll
+        for (int i = 0; i < S / 4; i++) {
+          const uint32_t x = ((w[i] >> (4 * (r >> 1))) & 0x0F0F0F0Fu) | (((u[i] >> (2 * r)) & 0x03030303u) << 4);
+#pragma unroll
+          for (int k = 0; k < 4; k++) o[g * S + 4 * i + k] = ds * (ubyte(x, k) - 32.f);
+        }
+      }
+    }
+  } else if constexpr (TAG == 12 || TAG == 13) {  // Q4_K, Q5_K (dequant.rs:385-444): d1 * q - m1
+    const int c = j >> 6, hi = (j >> 5) & 1, l = j & 31;
+    uint32_t sc, m;
+    scale_min_k4(2 * c + hi, b + 4, sc, m);
+    const float d1 = rd_f16(b, 0) * static_cast<float>(sc), m1 = rd_f16(b, 2) * static_cast<float>(m);
+    uint32_t w[N / 4];
+    rd_words<N, (N < 16 ? N : 16)>(b + (TAG == 12 ? 16 : 48) + 32 * c + l, w);
+#pragma unroll
+    for (int i = 0; i < N / 4; i++) w[i] = (w[i] >> (4 * hi)) & 0x0F0F0F0Fu;
+    if constexpr (TAG == 13) {  // fifth bits: bit 2c + hi of byte l
+      uint32_t h[N / 4];
+      rd_words<N, (N < 16 ? N : 16)>(b + 16 + l, h);
+#pragma unroll
+      for (int i = 0; i < N / 4; i++) w[i] |= ((h[i] >> (2 * c + hi)) & 0x01010101u) << 4;
+    }
+#pragma unroll
+    for (int e = 0; e < N; e++) v[e] = d1 * ubyte(w[e >> 2], e & 3) - m1;
+  } else if constexpr (TAG == 20) {  // IQ4_NL (dequant.rs:472-479)
+    const float d = rd_f16(b, 0);
+    nibbles16<N, 2>(b + 2, j, [&](int i, uint32_t w) {
+      const uint32_t x = iq4nl_values(w);
+#pragma unroll
+      for (int k = 0; k < 4; k++) v[4 * i + k] = d * sbyte(x, k);
+    });
+  } else if constexpr (TAG == 23) {  // IQ4_XS (dequant.rs:481-497)
+    const int ib = j >> 5;
+    const int ls = static_cast<int>(((b[4 + (ib >> 1)] >> (4 * (ib & 1))) & 0xFu) | (((rd_u16(b + 2) >> (2 * ib)) & 3u) << 4));
+    const float dl = rd_f16(b, 0) * static_cast<float>(ls - 32);
+    nibbles16<N, 8>(b + 8 + 16 * ib, j & 31, [&](int i, uint32_t w) {
+      const uint32_t x = iq4nl_values(w);
+#pragma unroll
+      for (int k = 0; k < 4; k++) v[4 * i + k] = dl * sbyte(x, k);
+    });
+  } else {
+#pragma unroll
+    for (int e = 0; e < N; e++) v[e] = decode<TAG>(b, j + e);
+  }
 }
 
 template <int TAG> struct Geo;

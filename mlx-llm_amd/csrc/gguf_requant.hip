@@ -6,10 +6,10 @@
 // (:156, as_dtype(bf16): round to nearest even) and the snapshot writer's
 // requant (:176 -> snapshot.rs:100-107 -> quant.rs:44, mlx quantize of the
 // bf16 tensor).  The reference materializes the whole f32 tensor on the host
-// and then the bf16 copy; here every lane gathers the 8 consecutive elements
-// of its output row straight from the GGUF blocks (un-permuted source row),
-// rounds them to bf16 and quantizes its share of the group in registers, so
-// the only HBM traffic is the GGUF bytes in and the packed MLX tensor out.
+// and then the bf16 copy; here every lane decodes consecutive elements of its
+// output row straight from the GGUF blocks (un-permuted source row), rounds
+// them to bf16 and quantizes its share of the group in registers, so the only
+// HBM traffic is the GGUF bytes in and the packed MLX tensor out.
 //
 // Bit-exactness: the element decode (gguf_decode.hpp) and the group
 // quantization (affine_group.hpp) are the ones of mlxq_gguf_dequantize and
@@ -27,19 +27,8 @@ namespace mlxq {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kEpl = 16;  // elements per lane
-
-// Element e of a float-typed GGUF tensor (F32 = 0, F16 = 1, BF16 = 30).
-template <int TAG>
-__device__ __forceinline__ float float_elem(const uint8_t* d, int64_t e) {
-  if constexpr (TAG == 0) {
-    return __uint_as_float(rd_u32(d + 4 * e));
-  } else if constexpr (TAG == 1) {
-    return f16_bits_to_f32(static_cast<uint32_t>(d[2 * e]) | (static_cast<uint32_t>(d[2 * e + 1]) << 8));
-  } else {
-    return bf16_bits_to_f32(static_cast<uint32_t>(d[2 * e]) | (static_cast<uint32_t>(d[2 * e + 1]) << 8));
-  }
-}
+constexpr int kUnit = 32;  // block formats: elements per lane
+constexpr int kFloatUnit = 16;  // float tensors: elements per lane
 
 template <int TAG>
 constexpr bool is_float_tag() {
@@ -62,122 +51,62 @@ __device__ __forceinline__ int source_row(int r, int perm_hd) {
   return h * perm_hd + 2 * (rr % half) + rr / half;
 }
 
-// The 16 consecutive elements j0 .. j0 + 15 (j0 a multiple of 16) of the
-// block at b (LDS), with the per-element arithmetic of decode<TAG> in the
-// same order (bit-identical), for the formats where one lane's 16 elements
-// share their bytes' layout: one nibble half of 16 consecutive bytes and one
-// scale.  decode<TAG> takes j at run time, so per element it re-derives the
-// half, the byte and (k-quants) the sub-block scale; here they are derived
-// once per lane and the bytes are read as whole 2- or 16-byte words.
-__device__ __forceinline__ uint32_t lds_u16(const uint8_t* p) { return *reinterpret_cast<const uint16_t*>(p); }
-
-template <int TAG>
-__device__ __forceinline__ void decode16(const uint8_t* b, int j0, float (&v)[kEpl]) {
-  if constexpr (TAG == 2 || TAG == 20) {
-    // Q4_0 / IQ4_NL: element j0 + k is nibble (j0 / 16) of byte 2 + k
-    const float d = rd_f16(b, 0);
-    const int sh = (j0 >> 2) & 4;
+// as_dtype(bf16): v_cvt_pk_bf16_f32, round to nearest even (a NaN payload
+// cannot reach a code: max/min skip NaN and a NaN quotient clamps to 0)
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+template <int N>
+__device__ __forceinline__ void round_bf16(float (&v)[N]) {
 #pragma unroll
-    for (int k = 0; k < 16; k += 2) {
-      const uint32_t w = lds_u16(b + 2 + k);
-      const uint32_t q0 = (w >> sh) & 0xFu, q1 = (w >> (sh + 8)) & 0xFu;
-      if constexpr (TAG == 2) {
-        v[k] = static_cast<float>(static_cast<int>(q0) - 8) * d;
-        v[k + 1] = static_cast<float>(static_cast<int>(q1) - 8) * d;
-      } else {
-        v[k] = d * static_cast<float>(iq4nl_value(q0));
-        v[k + 1] = d * static_cast<float>(iq4nl_value(q1));
-      }
-    }
-  } else if constexpr (TAG == 8) {
-    // Q8_0: element j0 + k is the signed byte 2 + j0 + k
-    const float d = rd_f16(b, 0);
-#pragma unroll
-    for (int k = 0; k < 16; k += 2) {
-      const uint32_t w = lds_u16(b + 2 + j0 + k);
-      v[k] = static_cast<float>(static_cast<int8_t>(w & 0xFFu)) * d;
-      v[k + 1] = static_cast<float>(static_cast<int8_t>(w >> 8)) * d;
-    }
-  } else if constexpr (TAG == 12) {
-    // Q4_K: sub-block 2c + hi; bytes 16 + 32c + (j0 & 31) .. +15 (16-byte aligned)
-    const int c = j0 >> 6, hi = (j0 >> 5) & 1;
-    uint32_t sc, m;
-    scale_min_k4(2 * c + hi, b + 4, sc, m);
-    const float d = rd_f16(b, 0), dmin = rd_f16(b, 2);
-    const float d1 = d * static_cast<float>(sc);
-    const float m1 = dmin * static_cast<float>(m);
-    const uint4 q = *reinterpret_cast<const uint4*>(b + 16 + 32 * c + (j0 & 31));
-    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-    const int sh = 4 * hi;
-#pragma unroll
-    for (int k = 0; k < 16; k++) {
-      const uint32_t nib = (w[k >> 2] >> (8 * (k & 3) + sh)) & 0xFu;
-      v[k] = d1 * static_cast<float>(nib) - m1;
-    }
-  } else if constexpr (TAG == 14) {
-    // Q6_K: 128-half idx, quarter t, bytes l = (j0 & 31) + k of ql (at 32 (t & 1),
-    // nibble t / 2) and qh (2-bit field t); one scale per 16 elements
-    const int idx = j0 >> 7, t = (j0 >> 5) & 3, l0 = j0 & 31;
-    const uint8_t* qlp = b + 64 * idx + 32 * (t & 1) + l0;
-    const uint8_t* qhp = b + 128 + 32 * idx + l0;
-    const int sc = static_cast<int8_t>(b[192 + 8 * idx + (l0 >> 4) + 2 * t]);
-    const float ds = rd_f16(b, 208) * static_cast<float>(sc);
-    const int shl = 4 * (t >> 1), shh = 2 * t;
-#pragma unroll
-    for (int k = 0; k < 16; k += 2) {
-      const uint32_t wl = lds_u16(qlp + k), wh = lds_u16(qhp + k);
-#pragma unroll
-      for (int e = 0; e < 2; e++) {
-        const uint32_t lo = (wl >> (8 * e + shl)) & 0xFu, hb = (wh >> (8 * e + shh)) & 3u;
-        const int q = static_cast<int>(static_cast<int8_t>(lo | (hb << 4))) - 32;
-        v[k + e] = ds * static_cast<float>(q);
-      }
-    }
-  } else if constexpr (TAG == 23) {
-    // IQ4_XS: sub-block ib, nibble (j0 / 16) & 1 of bytes 8 + 16 ib .. +15 (8-byte aligned)
-    const int ib = j0 >> 5;
-    const float d = rd_f16(b, 0);
-    const uint32_t shw = static_cast<uint32_t>(b[2]) | (static_cast<uint32_t>(b[3]) << 8);
-    const int ls = static_cast<int>((b[4 + (ib >> 1)] >> (4 * (ib & 1))) & 0xFu) |
-                   static_cast<int>(((shw >> (2 * ib)) & 3u) << 4);
-    const float dl = d * static_cast<float>(ls - 32);
-    const uint2 q0 = *reinterpret_cast<const uint2*>(b + 8 + 16 * ib);
-    const uint2 q1 = *reinterpret_cast<const uint2*>(b + 16 + 16 * ib);
-    const uint32_t w[4] = {q0.x, q0.y, q1.x, q1.y};
-    const int sh = (j0 >> 2) & 4;
-#pragma unroll
-    for (int k = 0; k < 16; k++) {
-      const uint32_t nib = (w[k >> 2] >> (8 * (k & 3) + sh)) & 0xFu;
-      v[k] = dl * static_cast<float>(iq4nl_value(nib));
-    }
+  for (int i = 0; i < N; i += 2) {
+    const bf16x2_t t = {static_cast<__bf16>(v[i]), static_cast<__bf16>(v[i + 1])};
+    const uint32_t u = __builtin_bit_cast(uint32_t, t);
+    v[i] = bits_to_f32(u << 16);
+    v[i + 1] = bits_to_f32(u & 0xFFFF0000u);
   }
 }
-template <int TAG>
-constexpr bool has_decode16() {
-  return TAG == 2 || TAG == 8 || TAG == 12 || TAG == 14 || TAG == 20 || TAG == 23;
+
+// the words of a lane's codes (16-byte stores), and its group's scale and
+// bias from the group's first lane
+template <int BITS, int LPG, int EPL>
+__device__ __forceinline__ void store_group(const uint32_t (&words)[EPL * BITS / 32], float scale, float bias,
+                                            int64_t lane, uint32_t* wq, uint16_t* scales, uint16_t* biases) {
+  constexpr int W = EPL * BITS / 32;
+  if constexpr (W == 2) {
+    reinterpret_cast<uint2*>(wq)[lane] = make_uint2(words[0], words[1]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < W / 4; j++)
+      reinterpret_cast<uint4*>(wq)[lane * (W / 4) + j] =
+          make_uint4(words[4 * j], words[4 * j + 1], words[4 * j + 2], words[4 * j + 3]);
+  }
+  if ((threadIdx.x & (LPG - 1)) == 0) {
+    const int64_t g = lane / LPG;
+    scales[g] = static_cast<uint16_t>(f32_to_bf16_bits(scale));
+    biases[g] = static_cast<uint16_t>(f32_to_bf16_bits(bias));
+  }
 }
 
-// A workgroup converts `rpw` consecutive output rows.  All of their source
-// rows' GGUF bytes are requested up front (direct global -> LDS loads when
-// 16-byte aligned, so the bytes in flight per CU are those of every resident
-// workgroup's rows), then every lane decodes 16 consecutive elements of a row
-// from LDS, rounds them to bf16 and quantizes its share of the group.
-// Each lane takes kEpl = 16 elements (LPG lanes per group), so the
-// per-block header decode and the per-group scale arithmetic, which every
-// lane of a group repeats, are shared by twice as many elements as with 8.
-
-template <int TAG, int BITS, int LPG, bool ALIGNED16>
+// A workgroup converts `rpw` consecutive output rows of a block format.  All
+// of their source rows' GGUF bytes are requested up front (direct global ->
+// LDS loads when 16-byte aligned), then every lane decodes 32 consecutive
+// elements of a row from LDS, rounds them to bf16 and quantizes its share of
+// the group.  Bound by the VALU (about 16 instructions per element): a lane
+// repeats its block's header decode and its group's scale arithmetic, so 32
+// elements share them.  14336 x 4096 to Q4 g64, 16 elements per lane with a
+// generic decode -> here (us): Q4_0 45.1 -> 30.5, Q5_0 53.4 -> 32.8, Q8_0
+// 42.9 -> 31.5, Q2_K 46.1 -> 28.9, Q3_K 76.3 -> 33.9, Q4_K 48.4 -> 32.4, Q5_K
+// 55.1 -> 29.2, Q6_K 54.4 -> 34.1, IQ4_NL 48.2 -> 30.7, IQ4_XS 49.7 -> 31.6.
+template <int TAG, int BITS, int LPG>
 __global__ __launch_bounds__(kThreads) void gguf_requant_kernel(const uint8_t* __restrict__ data, int rows, int K,
-                                                                 int row_bytes, int perm_hd, int rpw,
-                                                                 uint32_t* __restrict__ wq,
+                                                                 int row_bytes, int perm_hd, int rpw, int aligned16,
+                                                                 float rcp_lpr, uint32_t* __restrict__ wq,
                                                                  uint16_t* __restrict__ scales,
                                                                  uint16_t* __restrict__ biases) {
   extern __shared__ __align__(16) uint8_t lds[];
-  const int lpr = K / kEpl;  // lanes (kEpl elements each) per row
   const int r0 = blockIdx.x * rpw;
   const int nr = min(rpw, rows - r0);
   const int tid = threadIdx.x;
-  if constexpr (ALIGNED16) {
+  if (aligned16) {
     const int n16 = row_bytes >> 4;
     const int pieces = (n16 + 63) >> 6;  // 1 KB wave loads per row
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -194,84 +123,103 @@ __global__ __launch_bounds__(kThreads) void gguf_requant_kernel(const uint8_t* _
     }
   }
   __syncthreads();
-  for (int i = 0; i < nr; i++) {
-    const int r = r0 + i;
-    const uint8_t* row = lds + i * row_bytes;
-    // lanes of the row in whole groups per pass (kThreads is a multiple of LPG
-    // and lpr of LPG, so a group's lanes are active together)
-    for (int l0 = 0; l0 < lpr; l0 += kThreads) {
-      const int l = l0 + tid;
-      const bool active = l < lpr;
-      float v[kEpl];
-#pragma unroll
-      for (int j = 0; j < kEpl; j++) v[j] = 0.f;
-      if (active) {
-        const int e = l * kEpl;
-        if constexpr (is_float_tag<TAG>()) {
-#pragma unroll
-          for (int j = 0; j < kEpl; j++) v[j] = float_elem<TAG>(row, e + j);
-        } else {
-          constexpr int E = Geo<TAG>::E, B = Geo<TAG>::B;
-          static_assert(E % kEpl == 0, "a lane's elements never straddle a block");
-          const int blk = e / E;
-          const uint8_t* b = row + blk * B;
-          if constexpr (has_decode16<TAG>()) {
-            decode16<TAG>(b, e - blk * E, v);
-          } else {
-#pragma unroll
-            for (int j = 0; j < kEpl; j++) v[j] = decode<TAG>(b, e - blk * E + j);
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < kEpl; j++) v[j] = static_cast<float>(static_cast<__bf16>(v[j]));  // as_dtype(bf16): v_cvt_pk_bf16_f32, round to nearest even (a NaN payload cannot reach a code: max/min skip NaN and a NaN quotient clamps to 0)
-      }
-      uint32_t words[kEpl * BITS / 32];
-      float scale, bias;
-      quantize_group<BITS, LPG, kEpl>(v, words, scale, bias);  // every lane of the group takes part
-      if (active) {
-        const int64_t lane = static_cast<int64_t>(r) * lpr + l;
-#pragma unroll
-        for (int j = 0; j < BITS / 4; j++)
-          reinterpret_cast<uint2*>(wq)[lane * (BITS / 4) + j] = make_uint2(words[2 * j], words[2 * j + 1]);
-        if ((l & (LPG - 1)) == 0) {
-          const int64_t g = lane / LPG;
-          scales[g] = static_cast<uint16_t>(f32_to_bf16_bits(scale));
-          biases[g] = static_cast<uint16_t>(f32_to_bf16_bits(bias));
-        }
-      }
-    }
+  // the rows' units in one run: a group's lanes are adjacent (units per row
+  // and kThreads are multiples of LPG), lanes past the end repeat the last
+  // unit and store nothing
+  constexpr int E = Geo<TAG>::E, B = Geo<TAG>::B;
+  const int lpr = K / kUnit, units = nr * lpr;
+  for (int u0 = 0; u0 < units; u0 += kThreads) {
+    const int u = min(u0 + tid, units - 1);
+    // u / lpr: below 2^20 the f32 quotient of u + 1/2 cannot cross an integer
+    const int i = static_cast<int>((static_cast<float>(u) + 0.5f) * rcp_lpr);
+    const int l = u - i * lpr;
+    const uint8_t* b = lds + i * row_bytes + (E == 32 ? l : l >> 3) * B;
+    float v[kUnit];
+    decode_run<TAG, kUnit>(b, E == 32 ? 0 : (l & 7) * kUnit, v);
+    round_bf16(v);
+    uint32_t words[kUnit * BITS / 32];
+    float scale, bias;
+    quantize_group<BITS, LPG, kUnit>(v, words, scale, bias);
+    if (u0 + tid < units)
+      store_group<BITS, LPG, kUnit>(words, scale, bias, static_cast<int64_t>(r0) * lpr + u, wq, scales, biases);
   }
 }
 
-// Rows per workgroup: as many as fit 32 KB of LDS (at most 8), so that a
-// CU's resident workgroups keep ~100 KB of GGUF bytes in flight.
-inline int rows_per_workgroup(int row_bytes) {
-  return std::max(1, std::min(8, (32 * 1024) / std::max(row_bytes, 1)));
-}
-
+// F32 / F16 / BF16 tensors: nothing is shared between lanes, so each lane
+// takes its 16 elements straight from global memory (any alignment).  Bound
+// by HBM; through LDS with a per-element decode -> here (us, 14336 x 4096 to
+// Q4 g64): F16 72.2 -> 30.5, BF16 41.8 -> 28.1, F32 54.6 -> 48.9.
 template <int TAG, int BITS, int LPG>
-int launch_lpg(int rows, int K, int row_bytes, int perm_hd, const uint8_t* d, uint32_t* wq, uint16_t* s,
-               uint16_t* b, hipStream_t st) {
-  const bool al = (reinterpret_cast<uintptr_t>(d) & 15u) == 0 && row_bytes % 16 == 0;
-  const int rpw = rows_per_workgroup(row_bytes);
-  const size_t lds = static_cast<size_t>(rpw) * row_bytes;
-  const dim3 grid(static_cast<unsigned>((rows + rpw - 1) / rpw));
-  auto kern = al ? gguf_requant_kernel<TAG, BITS, LPG, true> : gguf_requant_kernel<TAG, BITS, LPG, false>;
-  if (lds > 64 * 1024) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-    if (e != hipSuccess) return fail(MLXQ_ERR_DEVICE, std::string("gguf_requantize: LDS size: ") + hipGetErrorString(e));
+__global__ __launch_bounds__(kThreads) void float_requant_kernel(const uint8_t* __restrict__ data, int64_t n_lanes,
+                                                                  int lpr, int perm_hd, uint32_t* __restrict__ wq,
+                                                                  uint16_t* __restrict__ scales,
+                                                                  uint16_t* __restrict__ biases) {
+  constexpr int B = kFloatUnit * (TAG == 0 ? 4 : 2);  // source bytes per lane
+  const int64_t lane = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+  int64_t src = min(lane, n_lanes - 1);
+  if (perm_hd > 0) {
+    int64_t r;
+    if (n_lanes <= UINT32_MAX) r = static_cast<uint32_t>(src) / static_cast<uint32_t>(lpr);
+    else r = src / lpr;
+    src += (static_cast<int64_t>(source_row(static_cast<int>(r), perm_hd)) - r) * lpr;
   }
-  MLXQ_LAUNCH(kern, grid, dim3(kThreads), lds, st, d, rows, K, row_bytes, perm_hd, rpw, wq, s, b);
+  uint32_t w[B / 4];
+  __builtin_memcpy(w, data + src * B, B);
+  float v[kFloatUnit];
+#pragma unroll
+  for (int i = 0; i < kFloatUnit; i++) {
+    if constexpr (TAG == 0) v[i] = bits_to_f32(w[i]);
+    else if constexpr (TAG == 1) v[i] = f16_to_f32((w[i >> 1] >> (16 * (i & 1))) & 0xFFFFu);
+    else v[i] = bits_to_f32((i & 1) ? w[i >> 1] & 0xFFFF0000u : w[i >> 1] << 16);
+  }
+  if constexpr (TAG != 30) round_bf16(v);
+  uint32_t words[kFloatUnit * BITS / 32];
+  float scale, bias;
+  quantize_group<BITS, LPG, kFloatUnit>(v, words, scale, bias);
+  if (lane < n_lanes) store_group<BITS, LPG, kFloatUnit>(words, scale, bias, lane, wq, scales, biases);
+}
+
+// Rows per workgroup: one 32-element unit for each of the 256 threads, so
+// that a CU holds several workgroups in different phases and one's loads run
+// beside another's arithmetic (14336 x 4096, 2 rows against 8: Q4_K 32.4 /
+// 33.2 us, Q5_K 29.2 / 30.9, Q8_0 31.5 / 35.3; 16 rows: 35.8 / 38.7 / 35.4),
+// at most 32 KB of LDS.
+inline int rows_per_workgroup(int units_per_row, int row_bytes) {
+  return std::max(1, std::min(static_cast<int>(ceil_div(kThreads, units_per_row)), (32 * 1024) / std::max(row_bytes, 1)));
+}
+
+template <int TAG, int BITS, int GS>
+int launch_gs(int rows, int K, int row_bytes, int perm_hd, const uint8_t* d, uint32_t* wq, uint16_t* s, uint16_t* b,
+              hipStream_t st) {
+  if constexpr (is_float_tag<TAG>()) {
+    const int lpr = K / kFloatUnit;
+    const int64_t lanes = static_cast<int64_t>(rows) * lpr;
+    MLXQ_LAUNCH((float_requant_kernel<TAG, BITS, GS / kFloatUnit>), dim3(static_cast<unsigned>(ceil_div(lanes, kThreads))),
+                dim3(kThreads), 0, st, d, lanes, lpr, perm_hd, wq, s, b);
+  } else {
+    const bool al = (reinterpret_cast<uintptr_t>(d) & 15u) == 0 && row_bytes % 16 == 0;
+    const int rpw = rows_per_workgroup(K / kUnit, row_bytes);
+    const size_t lds = static_cast<size_t>(rpw) * row_bytes;
+    const dim3 grid(static_cast<unsigned>((rows + rpw - 1) / rpw));
+    auto kern = gguf_requant_kernel<TAG, BITS, GS / kUnit>;
+    if (lds > 64 * 1024) {
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+      if (e != hipSuccess)
+        return fail(MLXQ_ERR_DEVICE, std::string("gguf_requantize: LDS size: ") + hipGetErrorString(e));
+    }
+    MLXQ_LAUNCH(kern, grid, dim3(kThreads), lds, st, d, rows, K, row_bytes, perm_hd, rpw, static_cast<int>(al),
+                1.0f / static_cast<float>(K / kUnit), wq, s, b);
+  }
   return check_launch("gguf_requantize");
 }
 
 template <int TAG, int BITS>
 int launch_bits(int group_size, int rows, int K, int row_bytes, int perm_hd, const uint8_t* d, uint32_t* wq,
                 uint16_t* s, uint16_t* b, hipStream_t st) {
-  if (group_size == 32) return launch_lpg<TAG, BITS, 32 / kEpl>(rows, K, row_bytes, perm_hd, d, wq, s, b, st);
-  if (group_size == 64) return launch_lpg<TAG, BITS, 64 / kEpl>(rows, K, row_bytes, perm_hd, d, wq, s, b, st);
-  return launch_lpg<TAG, BITS, 128 / kEpl>(rows, K, row_bytes, perm_hd, d, wq, s, b, st);
+  if (group_size == 32) return launch_gs<TAG, BITS, 32>(rows, K, row_bytes, perm_hd, d, wq, s, b, st);
+  if (group_size == 64) return launch_gs<TAG, BITS, 64>(rows, K, row_bytes, perm_hd, d, wq, s, b, st);
+  return launch_gs<TAG, BITS, 128>(rows, K, row_bytes, perm_hd, d, wq, s, b, st);
 }
 
 template <int TAG>

@@ -89,3 +89,22 @@ def test_requantize_errors(torch_gpu):
         mlxq.gguf_requantize(9, d, 1, 32, 0, 32, 4)
     with pytest.raises(mlxq.MlxqError):  # odd head_dim
         mlxq.gguf_requantize(2, torch.zeros(18 * 6, dtype=torch.uint8, device="cuda"), 6, 32, 2, 32, 4)
+
+
+@pytest.mark.parametrize("name", list(TAGS))
+@pytest.mark.parametrize("rows,cols,heads", [(5, 768, 0), (37, 2304, 0), (24, 10240, 3)])
+@pytest.mark.parametrize("gs,bits,offset", [(32, 4, 0), (128, 8, 0), (64, 4, 2)])
+def test_requantize_partial_workgroups(torch_gpu, name, rows, cols, heads, gs, bits, offset):
+    """Row counts that leave a partial workgroup, units per row that are no
+    power of two, every group size, data that is not 16-byte aligned."""
+    import torch
+
+    tag = TAGS[name]
+    data = blocks(tag, rows, cols, 980 + tag)
+    buf = np.zeros(data.size + offset, np.uint8)
+    buf[offset:] = data
+    got = mlxq.gguf_requantize(tag, torch.from_numpy(buf).cuda()[offset:], rows, cols, heads, gs, bits)
+    torch.cuda.synchronize()
+    want = orc.gguf_requantize(tag, data, rows, cols, heads, gs, bits)
+    for g, w in zip(got, want):
+        assert np.array_equal(host(g), w)
