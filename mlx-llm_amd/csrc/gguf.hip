@@ -13,6 +13,7 @@
 // fused, and f16 scales are decoded with integer bit operations.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <string>
 
 #include "common.hpp"
@@ -128,23 +129,59 @@ __global__ __launch_bounds__(kThreads) void gguf_dequant_kernel(const uint8_t* _
   }
 }
 
-// F32 / F16 / BF16 pass-through (dequant.rs:174-188): one element per thread.
+// F32 / F16 / BF16 pass-through (dequant.rs:174-188): bound by HBM.  A unit
+// is one 16-byte store (4 f32 or 8 bf16 outputs); a workgroup covers kFloatU
+// runs of 256 units, every run's loads first, each wave instruction storing 1
+// KB contiguously (non-temporal: not read back).  The data and, for these
+// types, the output may have any alignment: unaligned vector accesses.  One
+// element per thread with byte loads took 127-147 us for 14336 x 4096 (us
+// here, f32 / bf16 out: F16 56.9 / 40.1, BF16 56.7 / 40.2, F32 78.2 / 60.0).
+constexpr int kFloatU = 2;
+typedef u32x4 u32x4_any __attribute__((aligned(1)));
+
 template <int TAG, bool BF16OUT>
 __global__ __launch_bounds__(kThreads) void gguf_float_kernel(const uint8_t* __restrict__ data, int64_t n,
-                                                               void* __restrict__ out) {
-  int64_t e = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  if (e >= n) return;
-  float v;
-  if (TAG == 0) {
-    uint32_t w;
-    __builtin_memcpy(&w, data + 4 * e, 4);
-    v = bits_to_f32(w);
-  } else {
-    uint32_t h = static_cast<uint32_t>(data[2 * e]) | (static_cast<uint32_t>(data[2 * e + 1]) << 8);
-    v = TAG == 1 ? f16_to_f32(h) : bf16_bits_to_f32(h);
+                                                               uint8_t* __restrict__ out) {
+  constexpr int E = BF16OUT ? 8 : 4;           // elements per unit
+  constexpr int SB = E * (TAG == 0 ? 4 : 2);   // source bytes per unit
+  auto value = [](const uint32_t (&w)[SB / 4], int i) -> float {
+    if constexpr (TAG == 0) return bits_to_f32(w[i]);
+    const uint32_t h = (w[i >> 1] >> (16 * (i & 1))) & 0xFFFFu;
+    return TAG == 1 ? f16_to_f32(h) : bf16_bits_to_f32(h);
+  };
+  const int64_t units = n / E, u0 = static_cast<int64_t>(blockIdx.x) * (kThreads * kFloatU) + threadIdx.x;
+  if (units > 0) {
+    uint32_t w[kFloatU][SB / 4];
+#pragma unroll
+    for (int j = 0; j < kFloatU; j++)
+      __builtin_memcpy(w[j], data + min(u0 + j * kThreads, units - 1) * SB, SB);  // clamped: no branch around the loads
+#pragma unroll
+    for (int j = 0; j < kFloatU; j++) {
+      const int64_t u = u0 + j * kThreads;
+      if (u >= units) break;
+      u32x4 o;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        if constexpr (BF16OUT) o[i] = f32_to_bf16_bits(value(w[j], 2 * i)) | (f32_to_bf16_bits(value(w[j], 2 * i + 1)) << 16);
+        else o[i] = __float_as_uint(value(w[j], i));
+      }
+      __builtin_nontemporal_store(o, reinterpret_cast<u32x4_any*>(out + u * 16));
+    }
   }
-  if constexpr (BF16OUT) static_cast<uint16_t*>(out)[e] = static_cast<uint16_t>(f32_to_bf16_bits(v));
-  else static_cast<float*>(out)[e] = v;
+  // the last n % E elements: one thread each of the first workgroup
+  const int64_t e = units * E + threadIdx.x;
+  if (blockIdx.x == 0 && e < n) {
+    constexpr int B = TAG == 0 ? 4 : 2;
+    uint32_t w[SB / 4] = {};
+    __builtin_memcpy(w, data + e * B, B);
+    const float v = value(w, 0);
+    if constexpr (BF16OUT) {
+      const uint16_t h = static_cast<uint16_t>(f32_to_bf16_bits(v));
+      __builtin_memcpy(out + e * 2, &h, 2);
+    } else {
+      __builtin_memcpy(out + e * 4, &v, 4);
+    }
+  }
 }
 
 template <int TAG, bool BF16OUT>
@@ -163,9 +200,10 @@ void launch_blocks(const uint8_t* data, int64_t nblocks, void* out, hipStream_t 
 
 template <int TAG, bool BF16OUT>
 void launch_float(const uint8_t* data, int64_t n, void* out, hipStream_t st) {
-  int64_t grid = ceil_div(n, static_cast<int64_t>(kThreads));
-  if (grid == 0) return;
-  MLXQ_LAUNCH((gguf_float_kernel<TAG, BF16OUT>), dim3(grid), dim3(kThreads), 0, st, data, n, out);
+  if (n == 0) return;
+  const int64_t units = n / (BF16OUT ? 8 : 4);
+  const int64_t grid = std::max<int64_t>(1, ceil_div(units, static_cast<int64_t>(kThreads) * kFloatU));
+  MLXQ_LAUNCH((gguf_float_kernel<TAG, BF16OUT>), dim3(grid), dim3(kThreads), 0, st, data, n, static_cast<uint8_t*>(out));
 }
 
 template <bool BF16OUT>

@@ -141,3 +141,28 @@ def test_random_blocks_any_f16_scale(torch_gpu, tag):
     bn = (want_bf16 & 0x7FFF) > 0x7F80
     assert np.array_equal((got_bf16 & 0x7FFF) > 0x7F80, bn)
     assert np.array_equal(got_bf16[~bn], want_bf16[~bn])
+
+
+@pytest.mark.parametrize("tag", [0, 1, 30])
+@pytest.mark.parametrize("n", [1, 3, 8, 1027, 65536, 65536 + 4093])
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("offset", [0, 1, 6])
+def test_float_passthrough_every_encoding(torch_gpu, tag, n, bf16, offset):
+    """All 16-bit patterns (NaN payloads too), element counts that leave a
+    tail of the 16-byte units, and input and output at any alignment."""
+    if tag == 0:
+        data = orc.normal(3, n).view(np.uint8).copy()
+        data.view(np.uint32)[:n // 3] = rng.integers(0, 2**32, n // 3, dtype=np.uint64).astype(np.uint32)
+    else:
+        data = np.arange(n, dtype=np.uint32).astype(np.uint16).view(np.uint8)
+    ref = orc.gguf_dequantize(tag, data, n)
+    buf = np.zeros(data.size + offset, np.uint8)
+    buf[offset:] = data
+    dt = torch_gpu.bfloat16 if bf16 else torch_gpu.float32
+    out = torch_gpu.zeros(n + 2, dtype=dt, device="cuda")
+    mlxq.gguf_dequantize(tag, dev(buf)[offset:], n, out=out[1:n + 1])
+    torch_gpu.cuda.synchronize()
+    got = host(out)
+    assert got[0] == 0 and got[-1] == 0
+    want = orc.f32_to_bf16(ref) if bf16 else ref.view(np.uint32)
+    assert np.array_equal(got[1:-1] if bf16 else got[1:-1].view(np.uint32), want)
