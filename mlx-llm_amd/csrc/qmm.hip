@@ -15,9 +15,9 @@
 //    VALU), in whole 128-byte lines: the memory path pays per line touched,
 //    so a 32-byte slice of a code row costs as much as a full line.
 //      - activations: the BM x 64 bf16 tile of one step (one line per row),
-//        two stages, requested one step ahead;
+//        four stages (128-row tiles) or two, requested that many steps ahead;
 //      - codes: 128 bytes of each of the 256 weight rows (4 steps at Q4, 2
-//        at Q8), two buffers;
+//        at Q8), two buffers, requested a few at a time over the steps;
 //      - scales and biases: 16 bytes per row and array (8 steps of groups),
 //        two buffers.
 //    Rows are stored with their 16-byte chunks permuted (chunk c of row r at
@@ -30,6 +30,13 @@
 //    activation fragment of sub-step j is the 16-byte chunk 4h + j of the
 //    row: both operands follow the same k order, which the MFMA sums over.
 //    No weight tile is written to LDS.
+//  * Measured (us, M = 2048 on 4096 x 14336, M = 512 and 1024 on 14336 x
+//    4096, Q4): 202.4, 67.2, 127.8 -> 192.9, 63.7, 118.4 with the mixed FMA
+//    decode, paired requests, one wait per sub-step, four activation stages
+//    and spread code requests (Q8 the same: 218.1 -> 211.2, 74.9 -> 71.9).
+//    256 MFMA streams of random data draw enough power to run at 1.8 GHz (18
+//    ns per MFMA, 13.6 on up to 128 CUs): 147 us of the 193; the decode costs
+//    about 25, the LDS reads and requests the rest.
 //  * Step k's MFMAs use the operands decoded during step k-1: the wave
 //    alternates one MFMA (32 cycles on the matrix core) with a few decode
 //    instructions and LDS reads, in a fixed per-step schedule.
@@ -52,6 +59,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int BK = 64;      // K per step
 constexpr int PERIOD = 8;   // steps per unrolled period (one scale batch)
@@ -69,7 +77,8 @@ struct QmmGeom {
   static constexpr int C_BYTES = BN * 128;
   static constexpr int SROW = GS == 32 ? 32 : 16;  // scale bytes per row per batch (and bias bytes)
   static constexpr int S_BYTES = BN * 2 * SROW;
-  static constexpr int A_OFF = 0, C_OFF = 2 * A_BYTES, S_OFF = C_OFF + 2 * C_BYTES;
+  static constexpr int AST = TM <= 4 ? 4 : 2;  // activation stages: as many as fit
+  static constexpr int A_OFF = 0, C_OFF = AST * A_BYTES, S_OFF = C_OFF + 2 * C_BYTES;
   static constexpr int LDS_BYTES = S_OFF + 2 * S_BYTES;
   // DMA instructions per wave: activations per step, codes / scales per batch
   static constexpr int A_DMA = A_BYTES / 1024 / WAVES;
@@ -80,12 +89,48 @@ struct QmmGeom {
                 "whole DMA chunks");
   static_assert(PERIOD % CB == 0, "code batches tile the period");
   static_assert(WM * WN == WAVES && TM % 2 == 0 && TN % 2 == 0, "wave grid");
-  static_assert(4 * TM * TN >= 3 * TM * TN + 2 + A_DMA && 4 * TM * TN >= C_DMA + S_DMA, "DMA slots");
+  // activation fragments: two register sets where they fit (128-row tiles)
+  static constexpr int ASETS = TM <= 4 ? 2 : 1;
+  // slot of the step boundary, where every activation read of the step has
+  // been issued: with two sets those of the last sub-step go out in the first
+  // TM slots of the third, with one at its end
+  static constexpr int BOUNDARY = ASETS == 2 ? 2 * TM * TN + TM + 2 : 3 * TM * TN + 1;
+  static_assert(A_DMA % 2 == 0 && C_DMA % 4 == 0, "DMA pairs");
   static_assert(LDS_BYTES <= 160 * 1024, "fits in LDS");
-  static_assert(CB >= 2, "a code batch is needed two boundaries after its request");
-  // DMA instructions a boundary issues after its activations: codes when a
-  // batch starts two steps later, scales at boundary 6 of the period
-  static constexpr int after(int b) { return ((b + 2) % CB == 0 ? C_DMA : 0) + (b == PERIOD - 2 ? S_DMA : 0); }
+  static_assert(CB == 2 || CB == 4, "code batch schedule");
+  // Requests of step u (mod PERIOD), in issue order: after its boundary the
+  // activations of step u + AST into the stage that the boundary freed; then,
+  // in the next step's first slots, pairs [c_lo, c_hi) of a code batch and the
+  // scale batch two periods on.  Batch b is last read right after boundary CB
+  // b + CB - 3, so its buffer is free from the next boundary on: batch b + 2
+  // is requested by steps 4b + 2 and 4b + 3 (Q4) or 2b (Q8).  Codes come from
+  // HBM: spread out, so that they do not fill the miss queues at once, and
+  // waited for three (Q4) or two (Q8) steps after their request.
+  static constexpr int mod(int u, int n) { return ((u % PERIOD) + PERIOD) % n; }
+  static constexpr int C_PAIRS = C_DMA / 2;
+  static constexpr int c_lo(int u) { return CB == 4 && mod(u, 4) == 3 ? C_PAIRS / 2 : 0; }
+  static constexpr int c_hi(int u) {
+    if (CB == 2) return mod(u, 2) == 0 ? C_PAIRS : 0;
+    return mod(u, 4) == 2 ? C_PAIRS / 2 : mod(u, 4) == 3 ? C_PAIRS : 0;
+  }
+  static constexpr int C_AHEAD = CB == 2 ? 4 : 8;  // step kt requests from batch (kt + C_AHEAD) / CB
+  static constexpr int s_num(int u) { return mod(u, PERIOD) == PERIOD - 2 ? S_DMA : 0; }
+  static constexpr int step_num(int u) { return A_DMA + 2 * (c_hi(u) - c_lo(u)) + s_num(u); }
+  // Requests that may still be in flight at boundary u: those issued after the
+  // activations of step u + 1 and, where step u + 2 opens a code batch, after
+  // that batch's last pair (scale batches are older than either).
+  static constexpr int in_flight(int u) {
+    int a = step_num(u + 1 - AST) - A_DMA;
+    for (int v = u + 2 - AST; v < u; v++) a += step_num(v);
+    if ((u + 2) % CB == 0) {
+      const int w = u - (CB == 2 ? 2 : 3);
+      int c = s_num(w);
+      for (int v = w + 1; v < u; v++) c += step_num(v);
+      a = c < a ? c : a;
+    }
+    return a;
+  }
+  static_assert(4 * TM * TN > BOUNDARY + A_DMA / 2 && BOUNDARY > 2 * C_PAIRS + S_DMA, "DMA slots");
 };
 
 // LDS DMA of 16 bytes per lane (global_load_lds_dwordx4): lane l's bytes
@@ -93,16 +138,25 @@ struct QmmGeom {
 // builtin: the builtin only emits the 64-bit per-lane address form, while
 // the SGPR-base form (wave-uniform base + 32-bit per-lane offset) carries
 // half the per-lane address data, which the issuing wave pays for.  Every
-// LDS DMA of this kernel goes through these two functions, so M0 (the LDS
+// LDS DMA of this kernel goes through these functions, so M0 (the LDS
 // destination) is only ever written here, right before its use; the caller
 // accounts for them in its own s_waitcnt vmcnt (the compiler does not count
 // inline assembly).
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void dma16_to_lds_sbase(const void* base, uint32_t off, unsigned char* lds) {
+// Two requests for consecutive KB of LDS: the instruction's offset moves the
+// LDS destination and the memory address alike, so one M0 serves both, and
+// off1 is the second request's offset less 1024 (from a base 1024 lower, so
+// that it cannot be negative).
+constexpr uint32_t kDmaBias = 1024;
+__device__ __forceinline__ void dma16x2_to_lds_sbase(const void* base, uint32_t off0, uint32_t off1,
+                                                     unsigned char* lds) {
   const uint32_t m0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds)));
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(m0)
-               : "memory", "m0");
+  asm volatile(
+      "s_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024" ::"v"(
+          off0),
+      "v"(off1), "s"(base), "s"(m0)
+      : "memory", "m0");
 }
 __device__ __forceinline__ void dma16_to_lds(const void* g, unsigned char* lds) {
   const uint32_t m0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds)));
@@ -116,7 +170,13 @@ __device__ __forceinline__ void wait_vm() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
 }
-__device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xC07F); }
+// ... with only the LDS counter limited to n
+template <int N>
+__device__ __forceinline__ void wait_lgkm() {
+  static_assert(N >= 0 && N < 16, "lgkmcnt range");
+  __builtin_amdgcn_s_waitcnt(0xC07F | (N << 8));
+}
+__device__ __forceinline__ void wait_lgkm0() { wait_lgkm<0>(); }
 
 // 16-byte chunk position of logical chunk c in 128-byte LDS row r is
 // c ^ swz(r): a bijection within the row under which rows 0..15 at one c
@@ -172,14 +232,14 @@ __global__ __launch_bounds__(256, 1) void qmm_kernel(const uint16_t* __restrict_
 #pragma unroll
   for (int i = 0; i < Gm::A_DMA; i++) {
     const int r = 8 * (wave * Gm::A_DMA + i) + (lane >> 3), c = (lane & 7) ^ swz(r);
-    a_off[i] = (static_cast<uint32_t>(min(m0 + r, M - 1)) * K + kb + 8 * c) * 2;
+    a_off[i] = (static_cast<uint32_t>(min(m0 + r, M - 1)) * K + kb + 8 * c) * 2 + (i & 1 ? 0 : kDmaBias);
   }
   // codes: the same row / chunk mapping over 128-byte code lines
   uint32_t c_off[Gm::C_DMA];
 #pragma unroll
   for (int i = 0; i < Gm::C_DMA; i++) {
     const int r = 8 * (wave * Gm::C_DMA + i) + (lane >> 3), c = (lane & 7) ^ swz(r);
-    c_off[i] = static_cast<uint32_t>(min(n0 + r, N - 1)) * row_bytes + kb * BITS / 8 + 16 * c;
+    c_off[i] = static_cast<uint32_t>(min(n0 + r, N - 1)) * row_bytes + kb * BITS / 8 + 16 * c + (i & 1 ? 0 : kDmaBias);
   }
   // scales / biases: per row [scales SROW bytes][biases SROW bytes]; lanes
   // (row, array, 16-byte part)
@@ -195,14 +255,14 @@ __global__ __launch_bounds__(256, 1) void qmm_kernel(const uint16_t* __restrict_
 
   // DMA of the activations of step kt / code batch c / scale batch sb into
   // stage / buffer `buf` (the index is clamped past the end, the buffer not)
-  // instruction i of this wave's share of a DMA
+  // pair i of this wave's share of a DMA (the offsets carry kDmaBias)
   auto dma_a1 = [&](int kt, int buf, int i) __attribute__((always_inline)) {
-    dma16_to_lds_sbase(reinterpret_cast<const char*>(x) + kt * (BK * 2), a_off[i],
-                 lds + Gm::A_OFF + buf * Gm::A_BYTES + (wave * Gm::A_DMA + i) * 1024);
+    dma16x2_to_lds_sbase(reinterpret_cast<const char*>(x) + kt * (BK * 2) - kDmaBias, a_off[2 * i], a_off[2 * i + 1],
+                         lds + Gm::A_OFF + buf * Gm::A_BYTES + (wave * Gm::A_DMA + 2 * i) * 1024);
   };
   auto dma_c1 = [&](int c, int buf, int i) __attribute__((always_inline)) {  // steps CB c .. CB c + CB - 1
-    dma16_to_lds_sbase(reinterpret_cast<const char*>(wq) + c * 128, c_off[i],
-                 lds + Gm::C_OFF + buf * Gm::C_BYTES + (wave * Gm::C_DMA + i) * 1024);
+    dma16x2_to_lds_sbase(reinterpret_cast<const char*>(wq) + c * 128 - kDmaBias, c_off[2 * i], c_off[2 * i + 1],
+                         lds + Gm::C_OFF + buf * Gm::C_BYTES + (wave * Gm::C_DMA + 2 * i) * 1024);
   };
   auto dma_s1 = [&](int sb, int buf, int i) __attribute__((always_inline)) {  // steps 8 sb .. 8 sb + 7
     // groups from 8 * floor(first group / 8): 16 bytes of 8 groups (GS = 128:
@@ -212,11 +272,11 @@ __global__ __launch_bounds__(256, 1) void qmm_kernel(const uint16_t* __restrict_
   };
   auto dma_a = [&](int kt, int buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < Gm::A_DMA; i++) dma_a1(kt, buf, i);
+    for (int i = 0; i < Gm::A_DMA / 2; i++) dma_a1(kt, buf, i);
   };
   auto dma_c = [&](int c, int buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < Gm::C_DMA; i++) dma_c1(c, buf, i);
+    for (int i = 0; i < Gm::C_DMA / 2; i++) dma_c1(c, buf, i);
   };
   auto dma_s = [&](int sb, int buf) __attribute__((always_inline)) {
 #pragma unroll
@@ -286,114 +346,165 @@ __global__ __launch_bounds__(256, 1) void qmm_kernel(const uint16_t* __restrict_
     return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(as + i * 32 * 128 + a_rd[j][i & 1]));
   };
   // Decode piece p (0..31) of raw codes into `dst`: word w = p / 4 (tile
-  // w / 4, sub-step w % 4), bf16 pair p % 4 of its operand.
+  // w / 4, sub-step w % 4), bf16 pair p % 4 of its operand.  A masked code in
+  // the low bits of a half word is the subnormal half q * 2^-24 (times 16 for
+  // a nibble in bits 4-7: still below 2^11 units, where halves are linear),
+  // which v_fma_mix_f32 takes as it is: with the scale times 2^24 (2^20) the
+  // product is the exact s * q, one instruction per code and one mask per
+  // two (scales of 2^103 and above would overflow there).
   float sc[TN], zz[TN], sc16[TN];
-  uint32_t lo = 0, hi = 0, d[4];
-  auto piece = [&](const Raw& r, auto pc, bf16x8 (&dst)[TN][4]) __attribute__((always_inline)) {
+  uint32_t h0 = 0, h1 = 0, h2 = 0, h3 = 0, d[4];
+  auto half = [](uint32_t w, int i) __attribute__((always_inline)) {
+    return static_cast<float>(__builtin_bit_cast(f16x2, w)[i]);
+  };
+  float f0 = 0.f, f1 = 0.f;
+  auto piece_fma = [&](const Raw& r, auto pc) __attribute__((always_inline)) {
     constexpr int p = decltype(pc)::value;
     constexpr int w = p >> 2, tt = w >> 2, jj = w & 3, pp = p & 3;
     if constexpr (jj == 0 && pp == 0) {
-      sc[tt] = __uint_as_float(r.s[tt] << 16);
+      const float s0 = __uint_as_float(r.s[tt] << 16);
       zz[tt] = __uint_as_float(r.z[tt] << 16);
-      sc16[tt] = sc[tt] * 0.0625f;
+      sc[tt] = s0 * 0x1p24f;
+      sc16[tt] = s0 * 0x1p20f;
     }
     if constexpr (BITS == 4) {
+      // halves (q0, q4), (q1, q5), (q2, q6), (q3, q7)
       if constexpr (pp == 0) {
-        // even codes in the bytes of lo, odd codes (x16) in the bytes of hi
-        lo = r.w[tt][jj] & 0x0F0F0F0Fu;
-        hi = r.w[tt][jj] & 0xF0F0F0F0u;
-        asm("" : "+v"(lo), "+v"(hi));  // keep the byte form (one v_cvt_f32_ubyte per code)
+        h0 = r.w[tt][jj] & 0x000F000Fu;
+        h1 = r.w[tt][jj] & 0x00F000F0u;
       }
-      d[pp] = pack_bf16(__builtin_fmaf(sc[tt], static_cast<float>((lo >> (8 * pp)) & 0xFFu), zz[tt]),
-                        __builtin_fmaf(sc16[tt], static_cast<float>((hi >> (8 * pp)) & 0xFFu), zz[tt]));
+      if constexpr (pp == 1) {
+        h2 = (r.w[tt][jj] >> 8) & 0x000F000Fu;
+        h3 = (r.w[tt][jj] >> 8) & 0x00F000F0u;
+      }
+      f0 = __builtin_fmaf(half(pp & 1 ? h2 : h0, pp >> 1), sc[tt], zz[tt]);
+      f1 = __builtin_fmaf(half(pp & 1 ? h3 : h1, pp >> 1), sc16[tt], zz[tt]);
     } else {
-      const uint32_t q = r.w[tt][2 * jj + (pp >> 1)];
-      const int b0 = 16 * (pp & 1);
-      d[pp] = pack_bf16(__builtin_fmaf(sc[tt], static_cast<float>((q >> b0) & 0xFFu), zz[tt]),
-                        __builtin_fmaf(sc[tt], static_cast<float>((q >> (b0 + 8)) & 0xFFu), zz[tt]));
+      // word v = pp / 2: halves (q0, q2), (q1, q3)
+      if constexpr ((pp & 1) == 0) {
+        h0 = r.w[tt][2 * jj + (pp >> 1)] & 0x00FF00FFu;
+        h1 = (r.w[tt][2 * jj + (pp >> 1)] >> 8) & 0x00FF00FFu;
+      }
+      f0 = __builtin_fmaf(half(h0, pp & 1), sc[tt], zz[tt]);
+      f1 = __builtin_fmaf(half(h1, pp & 1), sc[tt], zz[tt]);
     }
+  };
+  // The pair of piece p packed and, with the fourth, the operand assembled:
+  // issued one piece later (a convert right after the mixed FMA it reads costs
+  // a wait state).
+  auto piece_pack = [&](float g0, float g1, auto pc, bf16x8 (&dst)[TN][4]) __attribute__((always_inline)) {
+    constexpr int p = decltype(pc)::value;
+    constexpr int w = p >> 2, tt = w >> 2, jj = w & 3, pp = p & 3;
+    d[pp] = pack_bf16(g0, g1);
     if constexpr (pp == 3) dst[tt][jj] = __builtin_bit_cast(bf16x8, u32x4{d[0], d[1], d[2], d[3]});
   };
 
   // One K step (kt = k0 + u) as a fixed instruction schedule: slot s issues
-  // MFMA s (sub-step j = s / (TM TN), row tile i, column tile tt); after the
-  // last MFMA of row tile i the LDS read of its fragment for sub-step j + 1
-  // (for j = 3: the next step's first sub-step) into the same registers;
-  // then decode pieces of the next step's operands.  Each slot is fenced, so
-  // the wave alternates between the matrix core and the vector ALU.  In the
-  // last sub-step, once every activation read of the step has been issued,
-  // sits the step boundary: wait for this wave's DMA of the next step's
-  // activations, barrier, issue the DMA that the schedule places here, read
-  // the codes of the step after next.  With 256-row tiles the decode pieces
-  // all come before the boundary, so one set of raw-code registers serves
-  // (the boundary refills it); with 128-row tiles they spread over the whole
-  // step and the raw codes are double-buffered.
-  constexpr int S = 4 * TM * TN, NP = 4 * 4 * TN, BOUNDARY = 3 * TM * TN + 1;
+  // MFMA s (sub-step j = s / (TM TN), row tile i, column tile tt); the LDS
+  // reads of the next sub-step's activation fragments (for j = 3: the next
+  // step's first), with two register sets in the first TM slots of a sub-step
+  // (one wait per sub-step), with one after the last MFMA of each row tile
+  // (two waits); then decode pieces of the next step's operands.  Each slot is fenced, so the wave alternates between the
+  // matrix core and the vector ALU.  What bounds it is the issue rate of one
+  // wave per SIMD, about five cycles an instruction of any kind, so the loop
+  // is kept short: 7.2 instructions per MFMA at TM = 4 (9.2 with one wait per
+  // fragment, one M0 write per request and a convert per code).
+  // Once every activation read of the step has been issued, sits the step
+  // boundary: wait for this wave's DMA of the next
+  // step's activations, barrier, issue the DMA that the schedule places here,
+  // read the codes of the step after next.  With 256-row tiles the decode
+  // pieces all come before the boundary, so one set of raw-code registers
+  // serves (the boundary refills it); with 128-row tiles they spread over the
+  // whole step and the raw codes are double-buffered.
+  constexpr int S = 4 * TM * TN, NP = 4 * 4 * TN, BOUNDARY = Gm::BOUNDARY;
   constexpr bool ONE_RAW = NP <= BOUNDARY;
   constexpr int PIECE_SLOTS = ONE_RAW ? BOUNDARY : S;
   constexpr int NRAW = ONE_RAW ? 1 : 2;
+  constexpr int ASETS = Gm::ASETS, AST = Gm::AST;
   const int KTL = KT - 1;
   auto step = [&](int k0, auto uc, const bf16x8 (&cur)[TN][4], bf16x8 (&nxt)[TN][4], const Raw& rcur, Raw& rnext,
-                  bf16x8 (&a)[TM]) __attribute__((always_inline)) {
+                  bf16x8 (&a)[Gm::ASETS][TM]) __attribute__((always_inline)) {
     constexpr int u = decltype(uc)::value;
     const int kt = k0 + u;
-    const unsigned char* as = lds + Gm::A_OFF + (u & 1) * Gm::A_BYTES;
-    const unsigned char* an = lds + Gm::A_OFF + ((u + 1) & 1) * Gm::A_BYTES;
+    const unsigned char* as = lds + Gm::A_OFF + u % AST * Gm::A_BYTES;
+    const unsigned char* an = lds + Gm::A_OFF + (u + 1) % AST * Gm::A_BYTES;
     static_for<S>([&](auto sc_) __attribute__((always_inline)) {
       constexpr int s = decltype(sc_)::value;
       constexpr int j = s / (TM * TN), r = s % (TM * TN), i = r / TN, tt = r % TN;
       if constexpr (s == BOUNDARY) {
-        wait_lgkm0();  // this wave's reads of stage kt & 1 are done
-        // activations of step kt + 1 (issued at the previous boundary, before
-        // the codes / scales that boundary issued)
-        wait_vm<Gm::after((u + PERIOD - 1) % PERIOD)>();
+        wait_lgkm0();  // this wave's reads of step kt's stage are done
+        // activations of step kt + 1 and the codes and scales of step kt + 2
+        wait_vm<Gm::in_flight(u)>();
         __builtin_amdgcn_s_barrier();
         read_raw(k0, std::integral_constant<int, u + 2>{}, rnext);
         __builtin_amdgcn_sched_barrier(0);
       }
+      constexpr int TH = TM / 2 * TN;
+      if constexpr (ASETS == 2 ? r == 0 && j < 3 : r % TH == 0 && s < BOUNDARY) {
+        // this (half) sub-step's fragments; after the boundary, its wait covers them
+        if constexpr (ASETS == 2) wait_lgkm0();
+        else wait_lgkm<TM / 2>();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      constexpr int set = ASETS == 2 ? j & 1 : 0, other = ASETS == 2 ? (j + 1) & 1 : 0;
       // weights as the first operand: the output tile comes out transposed,
       // lane = activation row, 4 consecutive output columns per register quad
-      acc[i][tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur[tt][j], a[i], acc[i][tt], 0, 0, 0);
-      if constexpr (tt == TN - 1) a[i] = read_a(j < 3 ? as : an, (j + 1) & 3, i);
-      // DMA, one instruction per slot so the requests do not queue up
-      // behind each other: after the boundary the activations of step kt + 2
-      // into stage kt & 1 (read by every wave before the barrier); in the
-      // first slots, when the previous boundary scheduled them (after its
-      // activations), code batch (kt + 1) / CB + 1 (when step kt + 1 starts a
-      // batch) and scale batch (kt + 9) / 8 (at u = 7).  Past the end: the
-      // last step / batch again, into buffers nobody reads.
-      if constexpr (s > BOUNDARY && s <= BOUNDARY + Gm::A_DMA) dma_a1(min(kt + 2, KTL), u & 1, s - BOUNDARY - 1);
-      if constexpr (u > 0 && (u + 1) % CB == 0 && s < Gm::C_DMA)
-        dma_c1(min((kt + 1) / CB + 1, KTL / CB), ((u + 1) / CB + 1) & 1, s);
-      if constexpr (u == PERIOD - 1 && s >= Gm::C_DMA && s < Gm::C_DMA + Gm::S_DMA)
-        dma_s1(min((kt + 9) / PERIOD, KTL / PERIOD), (k0 / PERIOD) & 1, s - Gm::C_DMA);
+      acc[i][tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur[tt][j], a[set][i], acc[i][tt], 0, 0, 0);
+      if constexpr (ASETS == 2 ? r < TM : tt == TN - 1) {
+        constexpr int ri = ASETS == 2 ? r : i;
+        a[other][ri] = read_a(j < 3 ? as : an, (j + 1) & 3, ri);
+      }
+      // DMA: after the boundary the activations of step kt + AST into the
+      // stage of step kt (read by every wave before the barrier); in the
+      // first slots what step kt - 1 left to do (see QmmGeom): a pair every
+      // other slot, then the scales.  Past the end: the last step / batch
+      // again, into buffers nobody reads.
+      constexpr int up = (u + PERIOD - 1) % PERIOD, CP = Gm::c_hi(up) - Gm::c_lo(up);
+      if constexpr (s > BOUNDARY && s <= BOUNDARY + Gm::A_DMA / 2)
+        dma_a1(min(kt + AST, KTL), u % AST, s - BOUNDARY - 1);
+      if constexpr (s % 2 == 1 && s / 2 < CP)
+        dma_c1(min((kt - 1 + Gm::C_AHEAD) / CB, KTL / CB), (u + PERIOD - 1 + Gm::C_AHEAD) / CB & 1, Gm::c_lo(up) + s / 2);
+      if constexpr (s >= 2 * CP && s < 2 * CP + Gm::s_num(up))
+        dma_s1(min((kt - 1) / PERIOD + 2, KTL / PERIOD), (k0 / PERIOD) & 1, s - 2 * CP);
       // pieces p with p * PIECE_SLOTS / NP == s
       constexpr int P_LO = (s * NP + PIECE_SLOTS - 1) / PIECE_SLOTS;
       constexpr int P_HI = ((s + 1) * NP + PIECE_SLOTS - 1) / PIECE_SLOTS;
       static_for<(NP + PIECE_SLOTS - 1) / PIECE_SLOTS>([&](auto qc) __attribute__((always_inline)) {
         constexpr int p = P_LO + decltype(qc)::value;
-        if constexpr (p < P_HI && p < NP) piece(rcur, std::integral_constant<int, p>{}, nxt);
+        if constexpr (p < P_HI && p < NP) {
+          const float g0 = f0, g1 = f1;
+          piece_fma(rcur, std::integral_constant<int, p>{});
+          if constexpr (p > 0) piece_pack(g0, g1, std::integral_constant<int, p - 1>{}, nxt);
+        }
       });
+      // the last pair of the step
+      if constexpr (s == (PIECE_SLOTS < S ? PIECE_SLOTS : S - 1))
+        piece_pack(f0, f1, std::integral_constant<int, NP - 1>{}, nxt);
       __builtin_amdgcn_sched_barrier(0);
     });
   };
 
   // ---- prologue: code batches 0 and 1, scale batches 0 and 1, activations
-  // of steps 0 and 1; the operands of step 0 decoded here
-  bf16x8 a[TM];
+  // of the first AST steps; the operands of step 0 decoded here
+  bf16x8 a[ASETS][TM];
   Raw raw[NRAW];
   dma_c(0, 0);
   dma_s(0, 0);
-  dma_a(0, 0);
-  dma_c(min(1, KTL / CB), 1);
+#pragma unroll
+  for (int i = 0; i < AST; i++) dma_a(min(i, KTL), i);
+  // of code batch 1 what no step of the loop requests
+#pragma unroll
+  for (int i = 0; i < (CB == 4 ? Gm::C_PAIRS / 2 : Gm::C_PAIRS); i++) dma_c1(min(1, KTL / CB), 1, i);
   dma_s(min(1, KTL / PERIOD), 1);
-  dma_a(min(1, KTL), 1);
-  wait_vm<Gm::A_DMA + Gm::C_DMA + Gm::S_DMA>();
+  wait_vm<0>();  // all of them: the waits of the loop count its own requests only
   __builtin_amdgcn_s_barrier();
   read_raw(0, std::integral_constant<int, 0>{}, raw[0]);
 #pragma unroll
-  for (int i = 0; i < TM; i++) a[i] = read_a(lds + Gm::A_OFF, 0, i);
-  static_for<NP>([&](auto pc) __attribute__((always_inline)) { piece(raw[0], pc, bop[0]); });
+  for (int i = 0; i < TM; i++) a[0][i] = read_a(lds + Gm::A_OFF, 0, i);
+  static_for<NP>([&](auto pc) __attribute__((always_inline)) {
+    piece_fma(raw[0], pc);
+    piece_pack(f0, f1, pc, bop[0]);
+  });
   read_raw(0, std::integral_constant<int, 1>{}, raw[NRAW - 1]);
 
   for (int k0 = 0; k0 < KT; k0 += PERIOD) {
@@ -561,7 +672,7 @@ int launch_qmm(const uint16_t* x, int64_t M, const uint32_t* wq, const uint16_t*
                const uint16_t* bias, int64_t N, int64_t K, int group_size, int bits, uint16_t* y, void* workspace,
                size_t workspace_bytes, hipStream_t st) {
   // the DMA offsets are 32-bit byte offsets from the array bases
-  if (M * K * 2 >= (int64_t(1) << 32) || N * K * bits / 8 >= (int64_t(1) << 32) || !qmm_eligible(K, group_size))
+  if (M * K * 2 + kDmaBias >= (int64_t(1) << 32) || N * K * bits / 8 + kDmaBias >= (int64_t(1) << 32) || !qmm_eligible(K, group_size))
     return fail(MLXQ_ERR_UNSUPPORTED, "qmm: activations and codes must each be below 4 GiB, K a multiple of " +
                                           std::to_string(PERIOD * BK) + " and of 8 groups");
   const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);

@@ -140,6 +140,32 @@ def test_qmm_tile_configs(torch_gpu, monkeypatch, bits, gs, cfg, n):
     assert rel_err(run(x, wq, s, b, gs, bits, mlxq.ALGO_QMM, bias=bias), ref) <= TIGHT
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("cfg", [82, 42])
+@pytest.mark.parametrize("k,factor", [(1024, 1.0), (2048, 2.0**-60), (3072, 2.0**60)])
+def test_qmm_decodes_every_weight_exactly(torch_gpu, monkeypatch, bits, gs, cfg, k, factor):
+    """One-hot activations: every output is one dequantized weight, which the
+    kernel rounds once from s * q + b, so y equals the dequantized matrix bit
+    for bit -- every code, every K step of one to three unrolled periods, and
+    scales far from 1."""
+    monkeypatch.setenv("MLXQ_QMM_CFG", str(cfg))
+    monkeypatch.setenv("MLXQ_QMM_SPLIT", "1")
+    n = 264
+    w = orc.f32_to_bf16((orc.normal(91 + bits + gs, n * k, 0, 0.02) * np.float32(factor)).astype(np.float32)).reshape(n, k)
+    wq, s, b = orc.affine_quantize(w, gs, bits, orc.BF16)
+    if factor < 1:  # the quantizer's smallest scale is 1e-7: scale the parameters instead
+        wq, s, b = make_layer(91 + bits + gs, n, k, gs, bits)
+        s, b = (orc.f32_to_bf16((orc.bf16_to_f32(t) * np.float32(factor)).astype(np.float32)).reshape(t.shape) for t in (s, b))
+    x = orc.f32_to_bf16(np.eye(k, dtype=np.float32)).reshape(k, k)
+    y = mlxq.qmatmul(dev(x, bf16=True), dev(wq), dev(s, bf16=True), dev(b, bf16=True), gs, bits, algo=mlxq.ALGO_QMM)
+    torch_gpu.cuda.synchronize()
+    want = orc.affine_dequantize(wq, s, b, gs, bits, orc.BF16).reshape(n, k).T
+    got = host(y)
+    zero = ((want | got) & 0x7FFF) == 0  # a zero weight may come out with either sign
+    assert np.array_equal(got[~zero], want[~zero])
+
+
 def test_bias_vector(torch_gpu):
     n, k = 192, 256
     wq, s, b = make_layer(70, n, k)
