@@ -174,10 +174,11 @@ int qmatmul_dispatch(const void* x, int64_t M, const uint32_t* wq, const void* s
   // tile kernel where qmv_tile_preferred says, the block kernel otherwise.
   // MLXQ_QMV_MFMA=1 never takes the vector-ALU kernel, MLXQ_QMV_DOT_ALL=1
   // takes it for every eligible M <= 4.
-  // whole rows per wave (qmv_row.hip) where K*bits/8 is a whole number of
+  // whole rows per wave (qmv_row.hip).  Where K*bits/8 is a whole number of
   // 1 KB load instructions: at M = 1, and at M = 2..4 for short matrices (N
   // <= 2048: k/v 6.1 -> 5.6 us Q4, 6.9 -> 5.1 Q8 at M = 4; on taller ones
-  // its per-row decode and LDS reads make it slower than the kernels below).
+  // its per-row decode and LDS reads make it slower than the kernels below);
+  // other rows where qmv_row_tail_preferred says.
   // MLXQ_QMV_NO_ROW=1 skips it, MLXQ_QMV_ROW_ALL=1 takes it for every M <= 4.
   const Overrides& ov = overrides();
   // M = 2: also on the taller matrices except Q4 gate/up-like ones (Q8 gate
@@ -185,7 +186,8 @@ int qmatmul_dispatch(const void* x, int64_t M, const uint32_t* wq, const void* s
   const bool gate_like = K < N && N * K >= (int64_t(1) << 25);
   // M = 3: Q8 gate/up-like ones too (19.42 -> 16.82 us; the other shapes at parity or slower)
   const bool row_m2 = (M == 2 && !(bits == 4 && gate_like)) || (M == 3 && bits == 8 && gate_like);
-  if (qmv_row_eligible(M, N, K, group_size, bits) && (M == 1 || row_m2 || N <= 2048 || ov.qmv_row_all) &&
+  const bool row = qmv_row_exact(K, bits) ? M == 1 || row_m2 || N <= 2048 : qmv_row_tail_preferred(M, N, K, bits);
+  if (qmv_row_eligible(M, N, K, group_size, bits) && (row || ov.qmv_row_all) &&
       !ov.qmv_no_row && !ov.qmv_mfma)
     return launch_qmv_row(xp, M, wq, sp, bp, bias, N, K, group_size, bits, yp, st);
   if (M <= kQmvDotMaxM && qmv_dot_eligible(M, N, K, group_size, bits) && !ov.qmv_mfma &&

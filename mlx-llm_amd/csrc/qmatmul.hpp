@@ -26,6 +26,10 @@ int launch_qmv(const QmvPlan& p, const uint16_t* x, int64_t M, const uint32_t* w
                hipStream_t st);
 
 // qmv_row: decode GEMV (M <= 4), whole rows per wave, 1 KB loads (qmv_row.hip).
+// qmv_row_exact: rows that the kernel reads without a tail (a whole number
+// of 1 KB loads with a form of its own).
+bool qmv_row_exact(int64_t K, int bits);
+bool qmv_row_tail_preferred(int64_t M, int64_t N, int64_t K, int bits);  // the other rows
 bool qmv_row_eligible(int64_t M, int64_t N, int64_t K, int group_size, int bits);
 int launch_qmv_row(const uint16_t* x, int64_t M, const uint32_t* wq, const uint16_t* s, const uint16_t* b,
                    const uint16_t* bias, int64_t N, int64_t K, int group_size, int bits, uint16_t* y,

@@ -71,6 +71,7 @@ struct RowParams {
   const uint16_t* norm_w;  // [K] RMSNorm weight (kNorm)
   float eps;
   int x_stride;
+  int K;                   // elements per row
   int gsh;                 // log2(group size)
   int rep_hd8, rep;        // kRepeat: head size in 8-element pieces, query heads per KV head
   float rcp_hd8, rcp_grp;  // 1 / rep_hd8, 1 / (rep_hd8 * rep)
@@ -108,18 +109,23 @@ __device__ __forceinline__ float bf16_round(float v) { return bf16_bits_to_f32(f
 //  * kSwiGLU (R = 2): a wave's two row slots are row n of the gate matrix
 //    and row n of the up matrix; y = bf16(bf16(g * bf16(sigmoid(g))) * u)
 //    with g, u the bf16 projection outputs (llama.rs:1040-1045).
-template <int BITS, int NI, int R, int W, int MM, int F>
+//  * TAIL: rows shorter than NI KB (any whole number of groups, p.K
+//    elements).  The lanes past the row repeat its last piece with zero
+//    activations, scale and bias (a bias that is not finite stays in its own
+//    group).
+template <int BITS, int NI, int R, int W, int MM, int F, bool TAIL>
 __global__ __launch_bounds__(64 * W) void qmv_row_kernel(const RowParams p) {
   constexpr int T = 64 * W;
-  constexpr int K = NI * 8192 / BITS;   // elements per row
+  constexpr int KP = NI * 8192 / BITS;  // elements per row, padded to whole loads
+  const int K = TAIL ? p.K : KP;        // elements per row
   constexpr int CPL = 128 / BITS;       // codes per lane per load (one chunk)
-  constexpr int NP = K / 8;             // 16-byte pieces of x
+  constexpr int NP = KP / 8;            // 16-byte pieces of x
   constexpr int XPT = (MM * NP + T - 1) / T; // pieces per thread (all activation rows)
   constexpr float OFF = BITS == 4 ? 128.f : 0.f;
   static_assert(NP % 4 == 0, "whole chunks of x");
   static_assert(!(F & kSwiGLU) || R == 2, "SwiGLU: a gate and an up row per wave");
   __shared__ uint4 xp[MM * NP];
-  __shared__ float xs[MM * (K / CPL)];
+  __shared__ float xs[MM * (KP / CPL)];
   __shared__ float ssq[(F & kNorm) ? W * MM : 1];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -145,7 +151,10 @@ __global__ __launch_bounds__(64 * W) void qmv_row_kernel(const RowParams p) {
 #pragma unroll
   for (int i = 0; i < XPT; i++) {
     const int q = min(tid + i * T, MM * NP - 1);  // clamped: no branch around the loads
-    const int m = q / NP, k8 = q - m * NP;
+    const int m = q / NP;
+    int k8 = q - m * NP;
+    const bool past = TAIL && k8 * 8 >= K;
+    if constexpr (TAIL) k8 = min(k8, K / 8 - 1);
     int src8 = k8;
     if constexpr (F & kRepeat) {
       const int grp = p.rep_hd8 * p.rep;
@@ -154,6 +163,7 @@ __global__ __launch_bounds__(64 * W) void qmv_row_kernel(const RowParams p) {
       src8 = hq * p.rep_hd8 + (r - div_rcp(r, p.rep_hd8, p.rcp_hd8) * p.rep_hd8);
     }
     xv[i] = *reinterpret_cast<const uint4*>(p.x + static_cast<int64_t>(m) * p.x_stride + src8 * 8);
+    if constexpr (TAIL) xv[i] = past ? make_uint4(0, 0, 0, 0) : xv[i];
     if constexpr (F & kNorm) nw[i] = reinterpret_cast<const uint4*>(p.norm_w)[k8];
   }
   // 2. the wave's rows: codes (1 KB per instruction), then the lanes' scale/bias
@@ -163,17 +173,18 @@ __global__ __launch_bounds__(64 * W) void qmv_row_kernel(const RowParams p) {
   for (int r = 0; r < R; r++) {
     const RowSeg& S = slot_seg(r);
     const int n = min(slot_row(r), S.N - 1);  // rows past N repeat row N-1 (results dropped)
-    const uint4* wr = reinterpret_cast<const uint4*>(S.wq) + static_cast<int64_t>(n) * (NI * 64);
+    const uint4* wr = reinterpret_cast<const uint4*>(S.wq) + static_cast<int64_t>(n) * (TAIL ? K * BITS / 128 : NI * 64);
+    auto piece = [&](int t) { return TAIL ? min(t * 64 + lane, K * BITS / 128 - 1) : t * 64 + lane; };
 #pragma unroll
     for (int t = 0; t < NI; t++) {
       if constexpr (NI <= 4) {
         // rows of up to 4 KB: non-temporal (the codes are read once; Q4 k
         // 3.36 -> 3.07 us, q 4.80 -> 4.62, Q8 q 5.81 -> 5.59); the 7 KB
         // rows of the down projection measured slower with it (9.9 -> 10.9)
-        const u32x4v q = __builtin_nontemporal_load(reinterpret_cast<const u32x4v*>(wr) + t * 64 + lane);
+        const u32x4v q = __builtin_nontemporal_load(reinterpret_cast<const u32x4v*>(wr) + piece(t));
         cw[r][t] = make_uint4(q.x, q.y, q.z, q.w);
       } else {
-        cw[r][t] = wr[t * 64 + lane];
+        cw[r][t] = wr[piece(t)];
       }
     }
   }
@@ -183,7 +194,7 @@ __global__ __launch_bounds__(64 * W) void qmv_row_kernel(const RowParams p) {
     const int n = min(slot_row(r), S.N - 1);
 #pragma unroll
     for (int t = 0; t < NI; t++) {
-      const int g = ((t * 64 + lane) * CPL) >> gsh;
+      const int g = TAIL ? min(((t * 64 + lane) * CPL) >> gsh, G - 1) : ((t * 64 + lane) * CPL) >> gsh;
       // non-temporal too (read once; Q4 k 3.03 -> 2.80 us, q 4.55 -> 4.28,
       // gate 8.9 -> 8.5-8.6, Q8 gate 13.8 -> 12.6-12.8), except for the Q4
       // 7 KB rows (down: 9.95-10.05 -> 10.05-10.26)
@@ -300,10 +311,11 @@ __global__ __launch_bounds__(64 * W) void qmv_row_kernel(const RowParams p) {
           decode_q8(wd[k], pr[2 * k], pr[2 * k + 1]);
         }
       }
-      const float s = bf16_bits_to_f32(sv[r][t]), b = bf16_bits_to_f32(bv[r][t]);
+      float s = bf16_bits_to_f32(sv[r][t]), b = bf16_bits_to_f32(bv[r][t]);
+      if (TAIL && t == NI - 1 && ch * CPL >= K) s = b = 0.f;
 #pragma unroll
       for (int m = 0; m < MM; m++) {
-        const float xsum = xs[m * (K / CPL) + ch];
+        const float xsum = xs[m * (KP / CPL) + ch];
         float d = 0.f;
         if (BITS == 4) {
           const uint4* xq = xp + m * NP + ch * 4;
@@ -367,9 +379,9 @@ __global__ __launch_bounds__(64 * W) void qmv_row_kernel(const RowParams p) {
   }
 }
 
-template <int BITS, int NI, int R, int W, int MM, int F>
+template <int BITS, int NI, int R, int W, int MM, int F, bool TAIL = false>
 int launch_rw(const RowParams& a, int64_t tiles, hipStream_t st) {
-  MLXQ_LAUNCH((qmv_row_kernel<BITS, NI, R, W, MM, F>), dim3(static_cast<unsigned>(tiles)), dim3(64 * W), 0, st,
+  MLXQ_LAUNCH((qmv_row_kernel<BITS, NI, R, W, MM, F, TAIL>), dim3(static_cast<unsigned>(tiles)), dim3(64 * W), 0, st,
                      a);
   return check_launch("qmv_row");
 }
@@ -417,6 +429,53 @@ int launch_ni(RowParams& a, int64_t M, int R, int W, hipStream_t st) {
   }
 }
 
+// Rows that are no whole number of 1 KB loads, or one with no exact form:
+// four waves per workgroup, one row per wave (two for short Q4 rows of tall
+// matrices).
+template <int BITS, int NI>
+int launch_tail(RowParams& a, int64_t M, int R, hipStream_t st) {
+  if constexpr (NI * 8192 / BITS <= 8192) {  // several activation rows: LDS
+    if (M >= 2 && M <= 4) {
+      const int64_t t = set_tiles(a, 1, 4, false);
+      if (M == 2) return launch_rw<BITS, NI, 1, 4, 2, 0, true>(a, t, st);
+      if (M == 3) return launch_rw<BITS, NI, 1, 4, 3, 0, true>(a, t, st);
+      return launch_rw<BITS, NI, 1, 4, 4, 0, true>(a, t, st);
+    }
+  }
+  if (M != 1) return fail(MLXQ_ERR_UNSUPPORTED, "qmv_row: M > 1 needs K <= 8192");
+  if constexpr (BITS == 4 && NI <= 3)
+    if (R >= 2) return launch_rw<BITS, NI, 2, 4, 1, 0, true>(a, set_tiles(a, 2, 4, false), st);
+  return launch_rw<BITS, NI, 1, 4, 1, 0, true>(a, set_tiles(a, 1, 4, false), st);
+}
+template <int BITS>
+int launch_tail_b(RowParams& a, int64_t ni, int64_t M, int R, hipStream_t st) {
+  switch (ni) {
+#define MLXQ_ROW_TAIL(NIV) \
+  case NIV:                \
+    return launch_tail<BITS, NIV>(a, M, R, st);
+    MLXQ_ROW_TAIL(1)
+    MLXQ_ROW_TAIL(2)
+    MLXQ_ROW_TAIL(3)
+    MLXQ_ROW_TAIL(4)
+    MLXQ_ROW_TAIL(5)
+    MLXQ_ROW_TAIL(6)
+    MLXQ_ROW_TAIL(7)
+    MLXQ_ROW_TAIL(8)
+    MLXQ_ROW_TAIL(9)
+    MLXQ_ROW_TAIL(10)
+    MLXQ_ROW_TAIL(11)
+    MLXQ_ROW_TAIL(12)
+    MLXQ_ROW_TAIL(13)
+    MLXQ_ROW_TAIL(14)
+#undef MLXQ_ROW_TAIL
+    default: return fail(MLXQ_ERR_UNSUPPORTED, "qmv_row: rows of at most 14 KB");
+  }
+}
+bool exact_ni(int64_t row_bytes) {
+  const int64_t ni = row_bytes / 1024;
+  return row_bytes % 1024 == 0 && (ni == 1 || ni == 2 || ni == 4 || ni == 7 || ni == 8 || ni == 14 || ni == 16);
+}
+
 // Fused forms at M = 1 (the batch-1 decode chain), K*bits/8 of 1, 2 or 4 KB.
 template <int BITS, int NI, int F>
 int launch_fused_r(RowParams& a, int R, hipStream_t st) {
@@ -459,28 +518,57 @@ int launch_fused_b(RowParams& a, int form, int64_t ni, int R, hipStream_t st) {
 
 }  // namespace row
 
+bool qmv_row_exact(int64_t K, int bits) { return row::exact_ni(K * bits / 8); }
+
 bool qmv_row_eligible(int64_t M, int64_t N, int64_t K, int group_size, int bits) {
   if (M < 1 || M > 4 || N < 1 || (bits != 4 && bits != 8) || group_size < 128 / bits) return false;
+  if (!qmv_row_exact(K, bits)) {  // with a tail
+    const int64_t ni = ceil_div(K * bits / 8, int64_t(1024));
+    return ni <= 14 && (M == 1 || ni * 8192 / bits <= 8192);
+  }
   if (M > 1 && K > 4096) return false;  // the activation rows share the workgroup's LDS
-  if ((K * bits / 8) % 1024) return false;
   const int64_t ni = K * bits / 8 / 1024;
   // Q4 with 7 KB rows (the down projection, K = 14336) run here, faster
   // than qmv_dot (9.92 -> 9.50 us at one row x 8 waves, less at two rows x
   // 4 waves); 14 KB and longer Q4 rows stay on qmv_dot
-  if (bits == 4 && ni >= 14 && !overrides().qmv_row_all) return false;
-  return ni == 1 || ni == 2 || ni == 4 || ni == 7 || ni == 8 || ni == 14 || ni == 16;
+  return !(bits == 4 && ni >= 14 && !overrides().qmv_row_all);
+}
+
+// Where rows with a tail run here by default (us, the other kernels -> here).
+//  * M = 1: from half a KB per row (below it most lanes idle: Q4 4096 x 768
+//    3.20 against 3.39).  Q4 5120 x 5120 8.3 -> 5.7, 13824 x 5120 13.1 ->
+//    10.5, 5120 x 13824 15.5 -> 11.2, 4096 x 11008 11.8 -> 8.8, 1024 x 5120
+//    5.3 -> 3.4, 2048 x 5632 5.3 -> 4.1, 14336 x 2304 9.6 -> 6.8; Q8 5120 x
+//    13824 25.1 -> 17.1, 13824 x 5120 21.4 -> 15.9, 32000 x 2560 26.2 -> 17.6.
+//    Q4 rows past 8 KB only where the matrix still gives each CU several
+//    workgroups of four rows (5120 x 17920 21.2 -> 15.4, 3584 x 18944 12.2
+//    against 12.9).
+//  * M = 2: rows of 3072 and more, except Q4 gate/up-like matrices (5120 x
+//    5120 Q4 11.2 -> 7.6, Q8 12.1 -> 9.1; Q8 16384 x 5120 26.0 -> 21.6; Q4 17.6
+//    against 19.6; 4096 x 2304 Q4 4.5 against 5.3).
+//  * M = 3 to 2048 rows of weights, M = 4 to 1024 (1024 x 5120 M = 4 Q4 6.7 ->
+//    5.3, Q8 6.8 -> 5.3; 2048 x 4608 Q4 6.5 against 6.8): each weight row
+//    reads every activation row from LDS.
+bool qmv_row_tail_preferred(int64_t M, int64_t N, int64_t K, int bits) {
+  if (M == 1) return K * bits / 8 >= 512 && !(bits == 4 && K > 16384 && N < 4096);
+  if (K < 3072) return false;
+  if (M == 2) return !(bits == 4 && K < N && N * K >= (int64_t(1) << 25));
+  return N <= (M == 3 ? 2048 : 1024);
 }
 
 // Rows per wave and waves per workgroup, from measurements at the Llama
 // shapes (MLXQ_QMV_ROW_R / MLXQ_QMV_ROW_W override them).
 void qmv_row_geometry(int64_t N, int64_t K, int bits, int& R, int& W) {
-  const int64_t ni = K * bits / 8 / 1024;
+  const int64_t ni = ceil_div(K * bits / 8, int64_t(1024));
   // Q4 gate 9.72 vs 10.48 us at 2 rows (with the non-temporal loads 8.4-8.8
   // either way); q/o 4.10 at 1 row vs 4.28 at 2 (it was 4.96 vs 5.18 the
   // other way before the non-temporal loads); Q4 down (7 KB rows) 10.06 us at
   // 2 rows x 4 waves against 10.66 at 1 x 8 and 11.16 at 2 x 8 (the two rows
   // share each lane's activation reads from LDS); Q8 best at 1
   R = bits == 4 && ((ni <= 2 && N > 8192) || ni == 7) ? 2 : 1;
+  // rows with a tail: 13824 x 5120 10.5 us at 2 rows, 10.9 at 1; 8192 x 3072
+  // 5.35 / 5.65; 5120 x 13824 12.25 / 11.2
+  if (!row::exact_ni(K * bits / 8)) R = bits == 4 && ni <= 3 && N >= 8192 ? 2 : 1;
   W = bits == 4 && ni >= 8 ? 8 : 4;  // Q8 down: 14.2 us at 4 waves, 16.9 at 8
   if (overrides().row_r) R = overrides().row_r;
   if (overrides().row_w) W = overrides().row_w;
@@ -493,6 +581,7 @@ row::RowParams row_params(const QmvFused& f) {
   a.norm_w = f.norm_w;
   a.eps = f.eps;
   a.x_stride = static_cast<int>(f.x_stride);
+  a.K = static_cast<int>(f.K);
   a.gsh = __builtin_ctz(static_cast<unsigned>(f.group_size));
   a.rep = f.rep > 1 ? f.rep : 1;
   a.rep_hd8 = f.rep > 1 ? f.rep_hd / 8 : 1;
@@ -523,6 +612,10 @@ int launch_qmv_row(const uint16_t* x, int64_t M, const uint32_t* wq, const uint1
   f.group_size = group_size;
   f.bits = bits;
   RowParams a = row_params(f);
+  if (!exact_ni(K * bits / 8)) {
+    const int64_t nt = ceil_div(K * bits / 8, int64_t(1024));
+    return bits == 4 ? launch_tail_b<4>(a, nt, M, R, st) : launch_tail_b<8>(a, nt, M, R, st);
+  }
 #define MLXQ_ROW_CASE(NIV)                                                  \
   case NIV:                                                                 \
     return bits == 4 ? launch_ni<4, NIV>(a, M, R, W, st) : launch_ni<8, NIV>(a, M, R, W, st);

@@ -384,6 +384,57 @@ def test_qmv_row_several_rows(torch_gpu, monkeypatch, bits, m, gs):
 
 
 @pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("gs", [32, 64, 128])
+def test_qmv_row_tail(torch_gpu, monkeypatch, bits, gs):
+    """The whole-row kernel on rows that are no whole number of 1 KB loads, at
+    M = 1 (one group past a load, 1.5 loads, five loads of Q8, the longest:
+    14 KB less a group; N below one workgroup, ragged, and tall enough for two
+    Q4 rows per wave) and forced with 2..4 activation rows; with a bias.  Bar:
+    TIGHT (bf16 output rounding)."""
+    per_kb = 8192 // bits
+    cases = [(1, n, k) for k in (per_kb + gs, 3072 if bits == 4 else 1536, 5120, 14 * per_kb - gs) for n in (8, 203)]
+    cases += [(1, 8203, 3072), (2, 203, 3072 + gs), (3, 203, 5120 - gs), (4, 203, 8192 - gs), (4, 8, per_kb + gs)]
+    monkeypatch.setenv("MLXQ_QMV_ROW_ALL", "1")
+    mlxq.reload_overrides()
+    for m, n, k in cases:
+        assert ", true>" in mlxq.qmatmul_route(m, n, k, gs, bits), (m, n, k)
+        wq, s, b = make_layer(0x80 + bits + gs + n, n, k, gs, bits)
+        x = bf16_acts(0x81 + m + k, m, k)
+        bias = orc.f32_to_bf16(np.linspace(-1, 1, n, dtype=np.float32))
+        ref = orc.qmatmul_f64(x, wq, s, b, gs, bits) + orc.bf16_to_f32(bias).astype(np.float64)[None, :]
+        assert rel_err(run(x, wq, s, b, gs, bits, bias=bias), ref) <= TIGHT, (m, n, k)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_qmv_row_tail_keeps_infinities_apart(torch_gpu, bits):
+    """An infinite bias in a row's last group makes that output infinite, not
+    NaN (the lanes past the row multiply nothing by it), and leaves the other
+    rows alone."""
+    n, k = 24, 1600
+    wq, s, b = make_layer(0x82, n, k, 64, bits)
+    x = orc.f32_to_bf16(np.abs(orc.bf16_to_f32(bf16_acts(0x83, 1, k))) + np.float32(0.5))
+    ref = orc.qmatmul_f64(x, wq, s, b, 64, bits)
+    b[5, -1] = 0x7F80
+    y = run(x, wq, s, b, 64, bits)
+    assert np.isposinf(y[0, 5])
+    rows = np.arange(n) != 5
+    assert rel_err(y[:, rows], ref[:, rows]) <= TIGHT
+
+
+def test_tail_row_routes(torch_gpu):
+    """Where rows with a tail take the whole-row kernel by default."""
+    r = mlxq.qmatmul_route
+    row = lambda m, n, k, bits: r(m, n, k, 64, bits).startswith("row::qmv_row_kernel")
+    assert row(1, 5120, 13824, 4) and row(1, 5120, 13824, 8) and row(1, 256, 1088, 4)
+    assert not row(1, 256, 960, 4) and row(1, 256, 576, 8) and not row(1, 256, 448, 8)
+    assert row(1, 4096, 17920, 4) and not row(1, 4095, 17920, 4) and not row(1, 4096, 14400, 8)
+    assert row(2, 5120, 5120, 4) and not row(2, 13824, 5120, 4) and row(2, 13824, 5120, 8)
+    assert row(2, 4096, 3136, 4) and not row(2, 4096, 3008, 4) and not row(2, 4096, 11008, 8)
+    assert row(3, 2048, 5632, 4) and not row(3, 2049, 5632, 4)
+    assert row(4, 1024, 5120, 8) and not row(4, 1025, 5120, 8)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("name,m", [("q_o", 128), ("q_o", 512), ("k_v", 256), ("down", 128), ("down", 256)])
 def test_qmm_small_grids_split_on_narrow_tiles(torch_gpu, bits, name, m):
     """The fused prefill kernel at grids that no split of 256 x 256 tiles
