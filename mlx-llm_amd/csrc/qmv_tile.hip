@@ -64,7 +64,7 @@ struct TileParams {
   float* part;  // [splits][M][N] partial sums (splits > 1)
   int M, N, K;
   int splits;
-  int steps;  // K slices per workgroup (streaming form)
+  int steps;  // K slices of the whole K, split over blockIdx.y (streaming form)
   // fused forms (whole-K form only, no K split): residual epilogue
   // y = bf16(res + bf16(acc + bias)); GQA head repeat by remapping the
   // activation loads; up to three weight matrices of the same activations,
@@ -632,7 +632,9 @@ __global__ __launch_bounds__(64 * WV) void qmv_stream_kernel(const TileParams p)
   __shared__ __align__(16) uint16_t sx[2][Tg::MR * Tg::SXS];
   __shared__ f32x4 red[KH > 1 ? (KH - 1) * Tg::RG * MT * 64 : 1];
   __shared__ f32x4 hand[SW ? Tg::RG / 2 * MT * 64 : 1];
-  const int steps = p.steps, s0 = blockIdx.y * steps, tile = blockIdx.x;
+  // slices [s0, s0 + steps) of the p.steps of K: as even as the split count allows
+  const int s0 = static_cast<int>(blockIdx.y) * p.steps / p.splits;
+  const int steps = (static_cast<int>(blockIdx.y) + 1) * p.steps / p.splits - s0, tile = blockIdx.x;
   // Every load below is issued on every path (a slice past the run re-reads
   // the last one): the memory counter then holds the same loads wherever
   // control flow joins, so each wait names exactly the loads it needs.  A
@@ -894,6 +896,15 @@ int run_stream(const TileParams& a, int tiles, int mblocks, hipStream_t st) {
   return check_launch("qmv_stream");
 }
 
+int cu_count() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 256;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) return 256;
+  return cus;
+}
+
+int64_t chunks_of(int64_t K, int bits) { return K * bits / 8 / 64; }
+
 // The streaming forms: (waves, Q4 chunks per wave and slice, K parts); Q8
 // takes twice the chunks, so a slice covers the same K either way.  Eight K
 // parts (one row group of 16 rows per workgroup, for short matrices) only
@@ -924,48 +935,6 @@ int dispatch_stream_mt(const SCfg& c, const TileParams& a, int tiles, int mb, hi
   return c.nch == 2 ? run_stream<BITS, MT, 8, 2 * F, 1>(a, tiles, mb, st)
                     : run_stream<BITS, MT, 8, 4 * F, 1>(a, tiles, mb, st);
 }
-// Where the streaming form is the default, from interleaved A/B timings
-// against the single-slice form at the Llama-3-8B shapes (weights streamed
-// from HBM, clocks warmed): large gate/up-like matrices (K < N) from M = 8:
-// Q4 M = 32 19.9 -> 17.4 us, Q8 24.3 -> 23.1, Q4 M = 16 14.5 -> 13.8, Q8 21.2
-// -> 19.5; down-like (K > N) with 4 K splits: M = 32 Q4 21.2 -> 19.6, Q8 25.8
-// -> 24.1, Q8 M = 16 23.1 -> 21.1 (Q4 M = 16 at parity).  The shorter
-// matrices (q/o, k/v) stay on the single-slice form (parity or slower).
-bool stream_preferred(int64_t M, int64_t N, int64_t K, int bits, SCfg& c, int& splits) {
-  const bool large = N * K >= (int64_t(1) << 25);
-  // gate/up-like from M = 3 (M = 4: Q4 13.20 -> 12.40 us, Q8 19.10 -> 18.47)
-  if (!large || M < (K < N ? 3 : 8)) return false;
-  // (re-measured with every load issued on every path: Q4 M = 32 gate 17.33
-  // -> 16.58 on {8, 2, 2}, Q8 M = 16 19.34 -> 18.41 on {4, 4, 1}, Q4 M = 16
-  // down 15.94 -> 15.56 on {4, 4, 1} with 4 splits)
-  if (K < N && N >= 65536) {
-    // very tall (an lm_head: 128256 rows, thousands of 64-row tiles): 4-wave
-    // workgroups, several per CU (Q4 M = 4 / 8 / 16 / 32: 85.6 / 91.5 /
-    // 95.6 / 119.8 -> 74.1 / 77.0 / 81.1 / 102.4 us; Q8 M = 4 132.0 -> 115.7,
-    // M = 32 161.3 -> 146.0 on {4, 2, 1})
-    c = bits == 8 && M > 16 ? SCfg{4, 2, 1} : SCfg{4, 4, 1};
-    splits = 1;
-    return true;
-  }
-  if (K < N) {
-    if (bits == 4) c = M > 16 || M <= 4 ? SCfg{8, 2, 2} : SCfg{8, 4, 2};
-    else c = M > 16 ? SCfg{8, 2, 2} : SCfg{4, 4, 1};  // Q8 M = 4 too: 18.44 -> 17.64 us against {8, 4, 2}
-    splits = 1;
-    return true;
-  }
-  if (M > 16) {
-    c = SCfg{8, 2, 2};
-    splits = 4;
-    return true;
-  }
-  if (M == 16 || (bits == 8 && M > 8)) {  // Q8 M = 9 / 12 / 15: 20.59 / 23.51 / 24.71 -> 19.56 / 19.79 / 19.76 us
-    c = SCfg{4, 4, 1};
-    splits = 4;
-    return true;
-  }
-  return false;
-}
-
 int dispatch_stream(int bits, int mt, const SCfg& c, const TileParams& a, int tiles, int mb, hipStream_t st) {
   if (bits == 4) return mt == 1 ? dispatch_stream_mt<4, 1>(c, a, tiles, mb, st) : dispatch_stream_mt<4, 2>(c, a, tiles, mb, st);
   return mt == 1 ? dispatch_stream_mt<8, 1>(c, a, tiles, mb, st) : dispatch_stream_mt<8, 2>(c, a, tiles, mb, st);
@@ -1009,15 +978,6 @@ int dispatch(int bits, const Cfg& c, const TileParams& a, int tiles, int mb, hip
   return c.mt == 1 ? run_wn<8, 1>(c, a, tiles, mb, st, q) : run_wn<8, 2>(c, a, tiles, mb, st, q);
 }
 
-int cu_count() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) return 256;
-  return cus;
-}
-
-int64_t chunks_of(int64_t K, int bits) { return K * bits / 8 / 64; }
-
 }  // namespace tile
 
 using namespace tile;
@@ -1051,13 +1011,103 @@ bool short_fullk(int64_t M, int64_t N, int64_t K, int bits, Cfg* c) {
   if (c) *c = f;
   return true;
 }
+
+// Streaming forms of shapes that the forms below cannot slice or leave a
+// part of the chip idle on (us, the kernel taken otherwise -> here).
+//  * Down-like (K > N) with eight K splits, as even as the slices divide, of
+//    4-wave workgroups, several per CU.  From 2^25 codes where the forms
+//    below (slices of 512 or 1024, four splits) do not divide K: Q4 5120 x
+//    13824 M = 4 / 8 / 16 / 32 24.0 / 29.6 / 38.5 / 62.8 -> 17.5 / 18.1 / 19.1
+//    / 24.0, 4096 x 11008 M = 8 / 16 / 32 14.4 / 18.2 / 27.3 -> 13.0 / 13.4 /
+//    16.2, 3584 x 18944 21.8 / 28.3 / 43.9 -> 18.1 / 18.5 / 22.4; Q8 5120 x
+//    13824 M = 4 / 8 / 32 28.2 / 33.4 / 66.0 -> 24.6 / 24.9 / 28.6, 4096 x
+//    11008 M = 12 / 32 17.9 / 28.1 -> 17.0 / 19.6.  (8192 x 28672, whose K they
+//    divide, M = 16 41.8 against 44.9.)  Below 2^25 codes while the
+//    workgroups are at most one per CU and the tile kernel's wide slices do
+//    not divide K: 2048 x 5632 Q4 M = 8 / 16 / 32 8.1 / 9.0 / 10.9 -> 6.9 /
+//    7.2 / 8.7, Q8 8.6 / 10.1 / 11.4 -> 7.8 / 8.2 / 9.8; 512 x 2816 M = 32 8.3
+//    -> 6.5 (M = 8 5.0 against 5.6); 2560 x 5632 Q8 M = 8 8.7 against 10.6.
+//  * Gate/up-like of 4097..8192 rows below 2^25 codes: 32-row tiles in one
+//    round of CUs.  8192 x 3072 Q4 M = 4 / 8 / 16 / 32 9.4 / 10.0 / 12.0 / 11.4
+//    -> 7.3 / 7.4 / 7.7 / 10.8, Q8 M = 8 / 16 / 32 9.5 / 11.5 / 14.0 -> 9.1 /
+//    9.7 / 12.6 (M = 3 / 4 8.4 / 8.6 against 8.9 / 9.1); 6144 x 4096 Q4 M = 4
+//    10.5 -> 8.7, Q8 M = 16 15.6 -> 11.2 (M = 32 14.0 against 14.7); 5632 x
+//    2048 Q8 M = 16 8.4 -> 7.1; 8192 x 1024 Q8 M = 8 4.6 against 5.2.
+bool stream_small(int64_t M, int64_t N, int64_t K, int bits, SCfg& c, int& splits) {
+  const bool large = N * K >= (int64_t(1) << 25);
+  const int64_t ch = chunks_of(K, bits);
+  if (K > N) {
+    const int64_t slices = K / 256;
+    const int64_t wgs = ceil_div(N, 64) * 8;  // with eight splits
+    if (K % 256) return false;
+    if (large) {
+      if (slices % 8 == 0 || M < (wgs > 2 * cu_count() ? 3 : bits == 4 ? 5 : 9)) return false;
+    } else if (wgs > cu_count() || ch % 16 == 0 || slices < 11 || M < (K >= 4096 ? 5 : 16)) {
+      return false;
+    }
+    c = large && M <= 16 && slices % 2 == 0 ? SCfg{4, 4, 1} : SCfg{4, 2, 1};
+    splits = 8;
+    return true;
+  }
+  if (K < N && !large && N > 4096 && N <= 8192 && K % 1024 == 0 && M >= (bits == 4 ? 3 : 6) &&
+      K >= (bits == 4 || M > 16 ? 3072 : 2048) && (M <= 16 || K < 4096) && !short_fullk(M, N, K, bits, nullptr)) {
+    c = SCfg{8, 2, 4};
+    splits = 1;
+    return true;
+  }
+  return false;
+}
+
+// Where the streaming form is the default, from interleaved A/B timings
+// against the single-slice form at the Llama-3-8B shapes (weights streamed
+// from HBM, clocks warmed): large gate/up-like matrices (K < N) from M = 8:
+// Q4 M = 32 19.9 -> 17.4 us, Q8 24.3 -> 23.1, Q4 M = 16 14.5 -> 13.8, Q8 21.2
+// -> 19.5; down-like (K > N) with 4 K splits: M = 32 Q4 21.2 -> 19.6, Q8 25.8
+// -> 24.1, Q8 M = 16 23.1 -> 21.1 (Q4 M = 16 at parity).  The shorter
+// matrices (q/o, k/v) stay on the single-slice form (parity or slower).
+bool stream_preferred(int64_t M, int64_t N, int64_t K, int bits, SCfg& c, int& splits) {
+  const bool large = N * K >= (int64_t(1) << 25);
+  if (stream_small(M, N, K, bits, c, splits)) return true;
+  // gate/up-like from M = 3 (M = 4: Q4 13.20 -> 12.40 us, Q8 19.10 -> 18.47)
+  if (!large || M < (K < N ? 3 : 8)) return false;
+  // (re-measured with every load issued on every path: Q4 M = 32 gate 17.33
+  // -> 16.58 on {8, 2, 2}, Q8 M = 16 19.34 -> 18.41 on {4, 4, 1}, Q4 M = 16
+  // down 15.94 -> 15.56 on {4, 4, 1} with 4 splits)
+  if (K < N && N >= 65536) {
+    // very tall (an lm_head: 128256 rows, thousands of 64-row tiles): 4-wave
+    // workgroups, several per CU (Q4 M = 4 / 8 / 16 / 32: 85.6 / 91.5 /
+    // 95.6 / 119.8 -> 74.1 / 77.0 / 81.1 / 102.4 us; Q8 M = 4 132.0 -> 115.7,
+    // M = 32 161.3 -> 146.0 on {4, 2, 1})
+    c = bits == 8 && M > 16 ? SCfg{4, 2, 1} : SCfg{4, 4, 1};
+    splits = 1;
+    return true;
+  }
+  if (K < N) {
+    if (bits == 4) c = M > 16 || M <= 4 ? SCfg{8, 2, 2} : SCfg{8, 4, 2};
+    else c = M > 16 ? SCfg{8, 2, 2} : SCfg{4, 4, 1};  // Q8 M = 4 too: 18.44 -> 17.64 us against {8, 4, 2}
+    splits = 1;
+    return true;
+  }
+  if (M > 16) {
+    c = SCfg{8, 2, 2};
+    splits = 4;
+    return true;
+  }
+  if (M == 16 || (bits == 8 && M > 8)) {  // Q8 M = 9 / 12 / 15: 20.59 / 23.51 / 24.71 -> 19.56 / 19.79 / 19.76 us
+    c = SCfg{4, 4, 1};
+    splits = 4;
+    return true;
+  }
+  return false;
+}
 }  // namespace
 
 bool qmv_tile_eligible(int64_t M, int64_t N, int64_t K, int group_size, int bits) {
   if (M < 1 || M > kQmvMaxM || N < 1 || group_size != 64) return false;
   if ((K * bits / 8) % 64) return false;
   const int64_t ch = chunks_of(K, bits);
-  if (ch % 4 || ch > 16 * kMaxSplits) return false;  // whole slices of 4, 8 or 16 chunks, <= 16 slices
+  // whole slices: of 4, 8 or 16 chunks, <= 16 slices, or of 2 (streaming form)
+  if (ch % 2 || ch > 16 * kMaxSplits) return false;
   return static_cast<int64_t>(kMaxSplits) * M * N < (int64_t(1) << 31);
 }
 
@@ -1106,7 +1156,7 @@ int launch_qmv_stream64(const uint16_t* x, int64_t M, const uint32_t* wq, const 
   a.N = static_cast<int>(N);
   a.K = static_cast<int>(K);
   a.splits = splits;
-  a.steps = static_cast<int>(K / 256 / splits);
+  a.steps = static_cast<int>(K / 256);
   a.part = splits > 1 ? static_cast<float*>(workspace) : nullptr;
   const int tiles = static_cast<int>(ceil_div(N, 16 * 8));
   const int mb = static_cast<int>(ceil_div(M, 64));
@@ -1116,6 +1166,9 @@ int launch_qmv_stream64(const uint16_t* x, int64_t M, const uint32_t* wq, const 
 }
 
 bool qmv_tile_preferred(int64_t M, int64_t N, int64_t K, int bits) {
+  SCfg c;
+  int splits = 1;
+  if (stream_small(M, N, K, bits, c, splits)) return true;
   // Measured against the block kernel (qmv.hip) and the vector-ALU kernel
   // (qmv_dot) at the Llama-3-8B projection shapes: the tile kernel wins on
   // the large projections from M = 8 (Q4) / 16 (Q8),
@@ -1125,6 +1178,18 @@ bool qmv_tile_preferred(int64_t M, int64_t N, int64_t K, int bits) {
   if (M <= 4) return large && K < N && M >= (bits == 4 ? 3 : 4);
   if (short_fullk(M, N, K, bits, nullptr)) return true;
   if (large) return K < N || M >= (bits == 4 ? 8 : 9);  // gate/up-like: the streaming form (Q8 M = 8 20.4 -> 19.0)
+  // Above 2^24 codes, unless the block kernel's 16-row workgroups fill its
+  // rounds of CUs (Q4: its only round): Q4 5120 x 5120 M = 5 / 8 / 16 12.4 /
+  // 14.5 / 17.8 -> 9.6 / 9.7 / 10.0 us, 3072 x 8192 M = 8 / 16 11.0 / 13.3 ->
+  // 9.1 / 9.4, 12288 x 2048 M = 8 9.6 -> 7.1; Q8 5120 x 5120 M = 8 / 16 13.9 /
+  // 17.9 -> 12.7 / 13.1, 9216 x 3072 M = 8 14.1 -> 12.0; filled: 4096 x 6144 M =
+  // 8 Q4 9.1 against 9.4, Q8 9.7 against 12.9, 12288 x 2048 Q8 10.9 against
+  // 11.1.  Q4 rows of one 2048-k slice: 5632 x 2048 M = 8 / 16 7.6 / 9.1 -> 5.1
+  // / 5.1.
+  const int64_t wgs = ceil_div(N, 16), cus = cu_count(), rounds = ceil_div(wgs, cus);
+  const bool full = wgs * 8 >= rounds * cus * 7;
+  if (N * K > (int64_t(1) << 24) && !(full && (bits == 8 || rounds == 1))) return M >= (bits == 4 ? 5 : 6);
+  if (bits == 4 && K == 2048 && N > 4096) return M >= 5;
   if (N <= 2048) return M >= 16;  // k/v: M = 16 Q4 8.28 -> 7.93 us, Q8 9.27 -> 8.06; Q8 M = 24 11.07 -> 8.93
   return M > 16;  // q/o-like: Q4 M = 20 10.16 -> 9.21 us, Q8 M = 24 11.36 -> 10.42 against the block kernel
 }
@@ -1173,10 +1238,10 @@ int launch_qmv_tile(const uint16_t* x, int64_t M, const uint32_t* wq, const uint
     // one M block of up to 32 rows, or (eight K parts, or MLXQ_QMV_TILE_MB)
     // blocks of 16
     const int mt = M <= 16 || c.kh == 8 || ov.tile_mb ? 1 : 2;
-    if (use && scfg_known(c, mt) && ch % per == 0 && (ch / per) % splits == 0 && splits <= kMaxSplits &&
+    if (use && scfg_known(c, mt) && ch % per == 0 && ch / per >= splits && splits <= kMaxSplits &&
         (splits == 1 || splits <= fit)) {
       a.splits = splits;
-      a.steps = static_cast<int>(ch / per / splits);
+      a.steps = static_cast<int>(ch / per);
       a.part = splits > 1 ? static_cast<float*>(workspace) : nullptr;
       const int64_t tiles = ceil_div(N, 16 * (c.wv / c.kh));
       const int mb = static_cast<int>(ceil_div(M, 16 * mt));
@@ -1196,14 +1261,15 @@ int launch_qmv_tile(const uint16_t* x, int64_t M, const uint32_t* wq, const uint
   // 25.6 -> 24.0 us, down 28.4 -> 25.7; Q4 M = 32 down 22.1 -> 20.8 against
   // one K part); q/o: Q8 M = 32 the same (12.7 -> 10.7 us), else 2 row
   // groups x 4 K parts of 4 chunks; k/v: that too (Q8 M = 32 8.5 -> 8.1 us)
-  // except Q4 M = 32, 4 waves, 4 chunks, one part.  Taken when it divides K
+  // except Q4 M = 32, 4 waves, 4 chunks, one part.  Above 2^24 codes as the
+  // large ones (Q4 M = 32 4096 x 6144 15.0 -> 11.4, 3072 x 8192 14.7 -> 11.3).
+  // Taken when it divides K
   // into at most 16 slices that fit the workspace, else the first such of
   // the others.
-  const bool large = N * K >= (int64_t(1) << 25);
   Cfg pref;
   pref.mt = M <= 16 || overrides().tile_mb ? 1 : 2;
   if (short_fullk(M, N, K, bits, &pref)) {
-  } else if (large || (bits == 8 && M > 16 && N > 2048)) {
+  } else if (N * K > (int64_t(1) << 24) || (bits == 8 && M > 16 && N > 2048)) {
     pref.wv = 8; pref.nch = 8; pref.kh = 2;
   } else if (N <= 2048 && bits == 4 && M > 16) {
     pref.wv = 4; pref.nch = 4; pref.kh = 1;

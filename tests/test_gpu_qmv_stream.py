@@ -58,6 +58,68 @@ def test_stream_configs(torch_gpu, stream, bits, cfg, k, m):
 
 
 @pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("cfg,k", [("4,2,1,8", 2048), ("4,2,1,8", 2816), ("4,2,1,8", 3840), ("4,4,1,8", 6656),
+                                   ("8,2,2,3", 4096), ("8,2,4,2", 3072)])
+@pytest.mark.parametrize("m", [5, 16, 17, 32])
+def test_stream_uneven_splits(torch_gpu, stream, bits, cfg, k, m):
+    """K splits that do not divide the slices: 8 over 8, 11, 13 and 15 slices
+    (K a multiple of 256 only), 3 over 8, 2 over 3."""
+    stream.setenv("MLXQ_QMV_TILE_STREAM", cfg)
+    n = 200
+    wq, s, b = make_layer(110 + bits, n, k, 64, bits)
+    x = bf16_acts(111 + m, m, k)
+    ref = orc.qmatmul_f64(x, wq, s, b, 64, bits)
+    assert rel_err(run(x, wq, s, b, 64, bits), ref) <= TIGHT
+
+
+# (bits, M, N, K, the kernel's name up to its activation-row blocks)
+ROUTES = [
+    (4, 3, 5120, 13824, "stream<4,64,1,4,4,1"), (4, 17, 5120, 13824, "stream<4,64,2,4,2,1"),
+    (8, 3, 5120, 13824, "stream<8,64,1,4,8,1"), (4, 4, 4096, 11008, "qmv_kernel"),
+    (4, 5, 4096, 11008, "stream<4,64,1,4,2,1"), (8, 8, 4096, 11008, "qmv_kernel"),
+    (8, 9, 4096, 11008, "stream<8,64,1,4,4,1"), (4, 5, 2048, 5632, "stream<4,64,1,4,2,1"),
+    (8, 32, 2048, 5632, "stream<8,64,2,4,4,1"), (8, 5, 2049, 5632, "qmv_kernel"),
+    (4, 15, 512, 2816, "qmv_kernel"), (4, 16, 512, 2816, "stream<4,64,1,4,2,1"),
+    (4, 3, 8192, 3072, "stream<4,64,1,8,2,4"), (4, 32, 8192, 3072, "stream<4,64,2,8,2,4"),
+    (8, 5, 8192, 3072, "qmv_kernel"), (8, 6, 8192, 3072, "stream<8,64,1,8,4,4"),
+    (8, 16, 4097, 2048, "stream<8,64,1,8,4,4"), (8, 17, 4097, 2048, "tile<8,64,2"),
+    (4, 5, 5120, 5120, "tile<4,64,1,8,8,1"), (8, 6, 5120, 5120, "tile<8,64,1,8,8,2"),
+    (4, 5, 5632, 2048, "tile<4,64,1,8,4,4"), (4, 32, 3072, 8192, "tile<4,64,2,8,8,2"),
+    (8, 6, 4096, 6144, "qmv_kernel"), (4, 8, 8192, 28672, "tile<4"),
+]
+
+
+@pytest.mark.parametrize("bits,m,n,k,kernel", ROUTES)
+def test_stream_and_tile_routes(torch_gpu, monkeypatch, bits, m, n, k, kernel):
+    """Both sides of each line of the default dispatch of batched decode away
+    from the Llama-3-8B shapes: the kernel's name, and (up to 2^25 codes; the
+    larger shapes run the same forms) sampled rows against the oracle."""
+    import mlxq
+    for v in ("MLXQ_QMV_TILE_STREAM", "MLXQ_QMV_TILE", "MLXQ_QMV_TILE_ALL"):
+        monkeypatch.delenv(v, raising=False)
+    mlxq.reload_overrides()
+    assert kernel in mlxq.qmatmul_route(m, n, k, 64, bits).replace(" ", "").replace("_kernel<", "<").replace(
+        "qmv<", "qmv_kernel<")
+    if n * k > 1 << 25:
+        return
+    wq, s, b = make_layer(0x120 + bits, n, k, 64, bits)
+    x = bf16_acts(0x121 + m, m, k)
+    y = run(x, wq, s, b, 64, bits)
+    rows = np.unique(np.concatenate([np.random.default_rng(0x122).choice(n, 128, replace=False), np.arange(n - 16, n)]))
+    assert rel_err(y[:, rows], orc.qmatmul_f64(x, wq[rows], s[rows], b[rows], 64, bits)) <= TIGHT
+
+
+def test_stream_splits_without_workspace(torch_gpu):
+    """Shapes whose default form splits K run on another kernel when the
+    workspace has no room for the partials."""
+    import mlxq
+    for bits, m, n, k in ((4, 8, 5120, 13824), (4, 8, 2048, 5632), (8, 16, 512, 2816), (4, 8, 5120, 5120)):
+        assert "split_reduce" in mlxq.qmatmul_route(m, n, k, 64, bits)
+        alone = mlxq.qmatmul_route(m, n, k, 64, bits, workspace_bytes=0)
+        assert "split_reduce" not in alone and "qmv" in alone, alone
+
+
+@pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("cfg", ["8,4,2,1", "8,2,2,4"])
 def test_stream_bias_and_outliers(torch_gpu, stream, bits, cfg):
     stream.setenv("MLXQ_QMV_TILE_STREAM", cfg)
