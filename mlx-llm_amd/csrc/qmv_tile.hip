@@ -1106,8 +1106,8 @@ bool qmv_tile_eligible(int64_t M, int64_t N, int64_t K, int group_size, int bits
   if (M < 1 || M > kQmvMaxM || N < 1 || group_size != 64) return false;
   if ((K * bits / 8) % 64) return false;
   const int64_t ch = chunks_of(K, bits);
-  // whole slices: of 4, 8 or 16 chunks, <= 16 slices, or of 2 (streaming form)
-  if (ch % 2 || ch > 16 * kMaxSplits) return false;
+  // whole slices: of 4, 8 or 16 chunks, <= 16 slices, or (the down-like streaming forms) of 2
+  if (ch % (K > N ? 2 : 4) || ch > 16 * kMaxSplits) return false;
   return static_cast<int64_t>(kMaxSplits) * M * N < (int64_t(1) << 31);
 }
 
