@@ -463,3 +463,32 @@ def test_route_query_names_the_kernels(torch_gpu):
     assert r(96, 14336, 4096, 64, 4, noalloc=True) == r(96, 14336, 4096, 64, 4)  # 64-row streaming form
     assert "split_reduce" in r(512, 4096, 4096, 64, 4)                           # qmm with K split
     assert r(512, 4096, 4096, 64, 4, workspace_bytes=0) == "qmm_kernel<4, 64, 4, 2>"  # no workspace: unsplit
+
+
+def test_calls_follow_the_current_stream(torch_gpu, monkeypatch):
+    """The raw stream handle that calls launch on is torch's current one: the
+    default stream, a side stream, and each thread's own; workspace_size()
+    follows reloaded overrides."""
+    import threading
+
+    import torch
+
+    cur = lambda: torch.cuda.current_stream().cuda_stream
+    assert mlxq._stream() == cur()
+    side = torch.cuda.Stream()
+    seen = []
+    with torch.cuda.stream(side):
+        assert mlxq._stream() == cur() == side.cuda_stream
+        t = threading.Thread(target=lambda: seen.append((mlxq._stream(), cur())))
+        t.start()
+        t.join()
+    assert seen[0][0] == seen[0][1] != side.cuda_stream
+    assert mlxq._stream() == cur() != side.cuda_stream
+    size = lambda: mlxq.workspace_size(100, 4096, 14336, 64, 4)
+    before = size()
+    monkeypatch.setenv("MLXQ_QMV_STREAM64", "1")
+    mlxq.reload_overrides()
+    assert size() == 4 * 100 * 4096 * 4 != before
+    monkeypatch.delenv("MLXQ_QMV_STREAM64")
+    mlxq.reload_overrides()
+    assert size() == before
