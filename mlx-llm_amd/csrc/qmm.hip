@@ -207,7 +207,8 @@ __global__ __launch_bounds__(256, 1) void qmm_kernel(const uint16_t* __restrict_
                                                      const uint16_t* __restrict__ scales,
                                                      const uint16_t* __restrict__ biases,
                                                      const uint16_t* __restrict__ bias_vec, int N, int K,
-                                                     uint16_t* __restrict__ y, float* __restrict__ part, int k_len) {
+                                                     uint16_t* __restrict__ y, float* __restrict__ part, int grain,
+                                                     int slice_grains, int longer) {
   using Gm = QmmGeom<BITS, GS, TM, TN>;
   constexpr int BM = Gm::BM, BN = Gm::BN, CB = Gm::CB;
   extern __shared__ __align__(16) unsigned char lds[];
@@ -221,8 +222,11 @@ __global__ __launch_bounds__(256, 1) void qmm_kernel(const uint16_t* __restrict_
   const int t = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
   if (t >= tiles) return;
   const int m0 = (t / nbn) * BM, n0 = (t % nbn) * BN;
-  const int kb = blockIdx.y * k_len;  // first K of this slice (split K)
-  const int KT = k_len / BK;          // a multiple of PERIOD
+  // split K: the first `longer` slices take slice_grains + 1 grains of K, the
+  // others slice_grains
+  const int sl = blockIdx.y;
+  const int kb = (sl * slice_grains + min(sl, longer)) * grain;            // first K of this slice
+  const int KT = (slice_grains + (sl < longer ? 1 : 0)) * (grain / BK);    // a multiple of PERIOD
   const int G = K / GS;
   const uint32_t row_bytes = static_cast<uint32_t>(K) * BITS / 8;
 
@@ -605,9 +609,10 @@ int launch(const uint16_t* x, int M, const uint32_t* wq, const uint16_t* s, cons
     attr_set = true;
   }
   const int64_t tiles = ceil_div(N, Gm::BN) * ceil_div(M, Gm::BM);
+  constexpr int grain = GS > PERIOD * BK / 8 ? 8 * GS : PERIOD * BK;
   dim3 grid(static_cast<unsigned>(8 * ceil_div(tiles, 8)), splits);
   MLXQ_LAUNCH(kern, grid, dim3(Gm::THREADS), Gm::LDS_BYTES, st, x, M, wq, s, b, bias, N, K, y,
-                     splits > 1 ? part : nullptr, K / splits);
+                     splits > 1 ? part : nullptr, grain, K / grain / splits, K / grain % splits);
   if (int rc = check_launch("qmm")) return rc;
   if (splits == 1) return MLXQ_OK;
   return launch_split_reduce(part, bias, y, M, N, splits, st);
@@ -648,19 +653,22 @@ bool qmm_eligible(int64_t K, int group_size) { return K % (PERIOD * BK) == 0 && 
 
 int qmm_split_k(int64_t M, int64_t N, int64_t K, int group_size) {
   // split K when even 128-row tiles leave most CUs idle; every slice is a
-  // whole number of unrolled periods and of 8-group scale batches.
+  // whole number of grains (unrolled periods and 8-group scale batches), as
+  // even as they divide: the fewest slices that make the longest one as short
+  // as one round of workgroups allows.  Against slices of one length, us: K =
+  // 5632 (11 grains, not split before) 2048 x 5632 M = 118 / 692 Q4 61.9 / 63.5
+  // -> 23.1 / 32.6, Q8 72.1 / 70.7 -> 25.3 / 36.7; K = 13824 (27) 5120 x 13824 M
+  // = 118 / 692 Q4 64.5 / 160 -> 39.6 / 114; K = 14336 (28) 4096 x 14336 M = 333
+  // 61.7 -> 58.0 (five slices for four); K = 5120 (10) 5120 x 5120 M = 333 44.1
+  // -> 36.9 (four for two).
   // MLXQ_QMM_SPLIT overrides (tests, tuning).
-  const int64_t grain = std::max<int64_t>(PERIOD * BK, 8 * group_size);
-  if (const int sp = overrides().qmm_split) {
-    return sp >= 1 && sp <= kQmmMaxSplits && K % (grain * sp) == 0 ? sp : 1;
-  }
+  const int64_t grains = K / std::max<int64_t>(PERIOD * BK, 8 * group_size);
+  if (const int sp = overrides().qmm_split) return sp >= 1 && sp <= kQmmMaxSplits && sp <= grains ? sp : 1;
   const int64_t cus = cu_count();
   const int64_t t128 = ceil_div(N, 256) * ceil_div(M, 128);
   if (t128 * 4 >= cus * 3) return 1;
-  int best = 1;
-  for (int sp = 2; sp <= kQmmMaxSplits; sp++)
-    if (t128 * sp <= cus && K % (grain * sp) == 0) best = sp;
-  return best;
+  const int64_t most = std::min(std::min<int64_t>(kQmmMaxSplits, grains), cus / t128);
+  return most > 1 ? static_cast<int>(ceil_div(grains, ceil_div(grains, most))) : 1;
 }
 
 size_t qmm_workspace_bytes(int64_t M, int64_t N, int64_t K, int group_size) {

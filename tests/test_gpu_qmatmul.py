@@ -435,6 +435,37 @@ def test_tail_row_routes(torch_gpu):
 
 
 @pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("gs,splits,k", [(32, 3, 2048), (64, 2, 1536), (64, 8, 5632), (128, 3, 5120), (128, 5, 6144)])
+def test_qmm_uneven_split_k(torch_gpu, monkeypatch, bits, gs, splits, k):
+    """qmm with K slices of two lengths (4 grains over 3, 3 over 2, 11 over 8,
+    5 over 3, 6 over 5; the grain is 512, 1024 at group size 128), ragged M
+    and N, both tile heights."""
+    monkeypatch.setenv("MLXQ_QMM_SPLIT", str(splits))
+    monkeypatch.setenv("MLXQ_QMM_FUSED", "1")
+    m, n = 300, 202
+    for cfg in ("42", "82"):
+        monkeypatch.setenv("MLXQ_QMM_CFG", cfg)
+        mlxq.reload_overrides()
+        assert mlxq.workspace_size(m, n, k, gs, bits) == splits * m * n * 4
+        wq, s, b = make_layer(0x94 + bits + gs, n, k, gs, bits)
+        x = bf16_acts(0x95 + splits, m, k)
+        ref = orc.qmatmul_f64(x, wq, s, b, gs, bits)
+        # as in test_qmm_split_k: the weights' bf16 rounding grows as sqrt(K)
+        assert rel_err(run(x, wq, s, b, gs, bits, mlxq.ALGO_QMM), ref) <= TIGHT * max(1, k / 4096) ** 0.5, cfg
+
+
+def test_qmm_split_counts(torch_gpu):
+    """The fewest slices that make the longest as short as one round allows."""
+    size = lambda m, n, k, gs=64: mlxq.workspace_size(m, n, k, gs, 4) / (4 * m * n)
+    assert size(333, 2048, 5632) == 6   # 11 grains: two each
+    assert size(333, 5120, 13824) == 4  # 27 grains, at most four slices of 60 tiles
+    assert size(333, 4096, 14336) == 5  # 28 grains, at most five of 48 tiles
+    assert size(512, 4096, 4096) == 4 and size(333, 1024, 4096) == 8
+    assert size(333, 1024, 5120, 128) == 5  # grains of 1024
+    assert size(2048, 4096, 14336) == 0
+
+
+@pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("name,m", [("q_o", 128), ("q_o", 512), ("k_v", 256), ("down", 128), ("down", 256)])
 def test_qmm_small_grids_split_on_narrow_tiles(torch_gpu, bits, name, m):
     """The fused prefill kernel at grids that no split of 256 x 256 tiles
