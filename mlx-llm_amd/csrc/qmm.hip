@@ -355,8 +355,9 @@ __global__ __launch_bounds__(256, 1) void qmm_kernel(const uint16_t* __restrict_
   // a nibble in bits 4-7: still below 2^11 units, where halves are linear),
   // which v_fma_mix_f32 takes as it is: with the scale times 2^24 (2^20) the
   // product is the exact s * q, one instruction per code and one mask per
-  // two (scales of 2^103 and above would overflow there).
+  // two (a scale of 2^104 and above overflows there: see the end of the loop).
   float sc[TN], zz[TN], sc16[TN];
+  float sc_max = 0.f;  // largest |sc| met (one v_max3_f32 per step; NaN does not count)
   uint32_t h0 = 0, h1 = 0, h2 = 0, h3 = 0, d[4];
   auto half = [](uint32_t w, int i) __attribute__((always_inline)) {
     return static_cast<float>(__builtin_bit_cast(f16x2, w)[i]);
@@ -370,6 +371,7 @@ __global__ __launch_bounds__(256, 1) void qmm_kernel(const uint16_t* __restrict_
       zz[tt] = __uint_as_float(r.z[tt] << 16);
       sc[tt] = s0 * 0x1p24f;
       sc16[tt] = s0 * 0x1p20f;
+      if constexpr (tt == TN - 1) sc_max = fmaxf(fmaxf(sc_max, fabsf(sc[0])), fabsf(sc[1]));
     }
     if constexpr (BITS == 4) {
       // halves (q0, q4), (q1, q5), (q2, q6), (q3, q7)
@@ -528,6 +530,69 @@ __global__ __launch_bounds__(256, 1) void qmm_kernel(const uint16_t* __restrict_
     });
   }
   wait_vm<0>();  // no DMA may land after the workgroup's LDS is released
+
+  // A finite scale of 2^104 and above became infinite in the decode's scaled
+  // multiply, and its weights infinite or (code 0) NaN.  A wave that met one
+  // forms its sums again with the unscaled multiply, in the same order, from
+  // global memory (never for weights of ordinary magnitude).
+  if (__builtin_expect(__any(sc_max == __builtin_inff()), 0)) {
+    static_assert(TN == 2, "a column per lane, sc[0] and sc[1]");
+    const uint16_t* sr = scales + static_cast<int64_t>(min(n0 + wn * 64 + lane, N - 1)) * G;
+    bool large = false;
+    for (int g = kb / GS; g < (kb + KT * BK) / GS; g++) {
+      const uint32_t e = sr[g] & 0x7FFFu;
+      large |= e >= 0x7380u && e < 0x7F80u;  // bf16 of 2^104; infinity
+    }
+    if (__any(large)) {
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int tt = 0; tt < TN; tt++)
+#pragma unroll
+          for (int v = 0; v < 16; v++) acc[i][tt][v] = 0.f;
+#pragma unroll 1
+      for (int kt = 0; kt < KT; kt++) {
+        const int k = kb + kt * BK + 32 * h;  // this lane's 32 k of the step
+        bf16x8 wv[TN][4];
+#pragma unroll
+        for (int tt = 0; tt < TN; tt++) {
+          const int64_t n = min(n0 + (wn * TN + tt) * 32 + fr, N - 1);
+          const float s0 = bf16_bits_to_f32(scales[n * G + k / GS]), z0 = bf16_bits_to_f32(biases[n * G + k / GS]);
+          const u32x4* wr = reinterpret_cast<const u32x4*>(wq) + (n * K + k) * BITS / 128;
+          uint32_t w[4 * Gm::CW];
+#pragma unroll
+          for (int v = 0; v < Gm::CW; v++) {
+            const u32x4 q = wr[v];
+#pragma unroll
+            for (int e = 0; e < 4; e++) w[4 * v + e] = q[e];
+          }
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            uint32_t o[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+              auto value = [&](int c) {  // code c of the lane's 32
+                const uint32_t q = (w[c * BITS / 32] >> (c * BITS % 32)) & ((1u << BITS) - 1);
+                return __builtin_fmaf(s0, static_cast<float>(q), z0);
+              };
+              o[e] = pack_bf16(value(8 * j + 2 * e), value(8 * j + 2 * e + 1));
+            }
+            wv[tt][j] = __builtin_bit_cast(bf16x8, u32x4{o[0], o[1], o[2], o[3]});
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+          for (int i = 0; i < TM; i++) {
+            const int64_t m = min(m0 + (wm * TM + i) * 32 + fr, M - 1);
+            const bf16x8 av = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(x + m * K + k + 8 * j));
+#pragma unroll
+            for (int tt = 0; tt < TN; tt++)
+              acc[i][tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[tt][j], av, acc[i][tt], 0, 0, 0);
+          }
+      }
+    }
+  }
 
   // Output layout of a 32x32 tile (weights x activations^T): lane holds
   // activation row m = lane % 32 and output columns n = 8 (v / 4) + 4 (lane /

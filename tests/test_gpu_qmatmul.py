@@ -385,6 +385,38 @@ def test_qmv_row_several_rows(torch_gpu, monkeypatch, bits, m, gs):
 
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("cfg,splits", [(82, 1), (42, 1), (42, 2)])
+def test_qmm_scales_up_to_the_largest(torch_gpu, monkeypatch, bits, gs, cfg, splits):
+    """One-hot activations over weights whose scales reach from 2^95 to 2^121
+    in some rows and single groups (2^104 and above do not fit the exponent
+    range of the decode's scaled multiply) and are ordinary elsewhere: y is
+    the dequantized matrix bit for bit, also next to a row with an infinite
+    scale; K in one slice and in two."""
+    monkeypatch.setenv("MLXQ_QMM_CFG", str(cfg))
+    monkeypatch.setenv("MLXQ_QMM_SPLIT", str(splits))
+    monkeypatch.setenv("MLXQ_QMM_FUSED", "1")
+    n, k = 517, 2048
+    wq, s, b = make_layer(0x97 + bits + gs, n, k, gs, bits)
+    exp = np.zeros((n, k // gs), np.int32)
+    exp[3:20] = np.arange(102, 119)[:, None]  # on scales of about 2^-7 (Q4) and 2^-11 (Q8)
+    exp[70, 1] = exp[100, -1] = exp[516, 3] = exp[300:320] = 120
+    s, b = (orc.f32_to_bf16(np.ldexp(orc.bf16_to_f32(t).reshape(n, -1), exp).astype(np.float32)).reshape(t.shape)
+            for t in (s, b))
+    s[33, 2] = 0x7F80
+    x = orc.f32_to_bf16(np.eye(k, dtype=np.float32)).reshape(k, k)
+    y = mlxq.qmatmul(dev(x, bf16=True), dev(wq), dev(s, bf16=True), dev(b, bf16=True), gs, bits, algo=mlxq.ALGO_QMM)
+    torch_gpu.cuda.synchronize()
+    want = orc.affine_dequantize(wq, s, b, gs, bits, orc.BF16).reshape(n, k).T
+    got = host(y)
+    keep = np.arange(n) != 33
+    assert not np.isfinite(orc.bf16_to_f32(got[:, 33])).any()
+    got, want = got[:, keep], want[:, keep]
+    zero = ((want | got) & 0x7FFF) == 0  # a zero weight may come out with either sign
+    assert np.array_equal(got[~zero], want[~zero])
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("gs", [32, 64, 128])
 def test_qmv_row_tail(torch_gpu, monkeypatch, bits, gs):
     """The whole-row kernel on rows that are no whole number of 1 KB loads, at
     M = 1 (one group past a load, 1.5 loads, five loads of Q8, the longest:
