@@ -21,9 +21,10 @@
 //    4 x 4 dword transpose across the lane rows gives group-pure MFMA
 //    blocks; P = sum x (OFF + q) per group, acc += s P in f32.  The rest of
 //    the affine term, sum_g S_g (b - OFF s) with S_g the group's sum of x,
-//    is one MFMA (two for Q4) per slice: the group sums are formed once per
-//    workgroup while staging (not per wave and chunk) and fed as bf16 hi/lo
-//    halves against the bf16 biases (and scales).
+//    is one MFMA (two for Q4; twice that for more than 8 groups) per slice:
+//    the group sums are formed once per workgroup while staging (not per wave
+//    and chunk) and fed as three bf16 parts, exact to all 24 bits, against
+//    the bf16 biases (and scales).
 //  * Split K: blockIdx.y picks the slice.  With more than one slice the
 //    workgroups store f32 partial tiles in the caller's workspace and a
 //    second, elementwise kernel adds them in slice order (deterministic),
@@ -155,10 +156,10 @@ struct TileGeom {
   static constexpr int NG = KS / GS;                 // groups per wave slice
   static constexpr int NGW = NG / 2;                 // parameter words per row and wave slice
   // group sums of the staged activations, as MFMA A operands of the bias
-  // term: per row and K part [hi(0..NGP), lo(0..NGP), zeros] in bf16, KB
-  // blocks of 32 k
+  // term: per row and K part [hi(0..NGP), mid(0..NGP), lo(0..NGP), zeros] in
+  // bf16, KB blocks of 32 k
   static constexpr int NGP = NG < 8 ? 8 : NG;        // groups padded to whole 8-lane slices
-  static constexpr int KB = (2 * NGP + 31) / 32;     // bias-term MFMAs per M tile
+  static constexpr int KB = (3 * NGP + 31) / 32;     // bias-term MFMAs per M tile
   static constexpr int SXP = 32 * KB;                // bf16 per K part
   static constexpr int SXS = KH * SXP + 8;           // bf16 per row (8 of padding)
   // codes loaded row-contiguous across lanes (tile_load_w)
@@ -168,12 +169,6 @@ struct TileGeom {
   static_assert(NG % 2 == 0 && (NGW == 2 || NGW % 4 == 0), "parameters load as whole vectors");
   static_assert(NGP % 8 == 0 && (KW / 8) % 8 == 0, "a group's eight pieces sit in eight consecutive lanes");
 };
-
-__device__ __forceinline__ uint32_t bf16_rne_bits(float f) {
-  uint32_t u = __float_as_uint(f);
-  u += 0x7FFFu + ((u >> 16) & 1u);
-  return u >> 16;
-}
 
 // One work item (16 RG weight rows x one workgroup K slice): its global
 // data, held in registers from the loads until they are used -- the
@@ -277,9 +272,15 @@ __device__ __forceinline__ void tile_stage(const TileX<BITS, GS, MT, WV, NCH, KH
   // permutation is done once here instead of by every wave per block.  The
   // sum of x over each group (row m, group g) is formed here once for the
   // workgroup: a piece's 8 values with v_dot2 against ones, then the group's
-  // 8 pieces (8 consecutive lanes) with DPP adds; it is stored as the bf16
-  // pair hi + lo (hi = bf16(S), lo = bf16(S - hi): S to about 2^-16).
+  // 8 pieces (8 consecutive lanes) with DPP adds; it is stored as three bf16
+  // parts that add up to it exactly (each the leading 8 bits, cut off, of
+  // what the ones before it leave of the 24; an infinity is its first part).
+  // All eight lanes hold the sum: lane j forms and stores part min(j, 2), one
+  // LDS store per piece (a Llama-3-8B layer, Q4 M = 32: 84.1 us; 86.3 with
+  // three stores by every lane, 84.0 with two parts, which kept 16 bits).
   const uint32_t one2 = 0x3F803F80u;  // bf16 (1, 1)
+  const int spart = min(tid & 7, 2);
+  const uint32_t cut1 = spart >= 1 ? 0xFFFF0000u : 0u, cut2 = spart >= 2 ? 0xFFFF0000u : 0u;
 #pragma unroll
   for (int i = 0; i < Tg::XP; i++) {
     float ps = 0.f;
@@ -298,19 +299,18 @@ __device__ __forceinline__ void tile_stage(const TileX<BITS, GS, MT, WV, NCH, KH
     } else {
       xs[row * Tg::ROW16 + col] = X.xg[i];
     }
-    // the group's 8 lanes store the same value (no branch)
+    const float r1 = ps - __uint_as_float(__float_as_uint(ps) & cut1);
+    const float r = fabsf(ps) == __builtin_inff() && spart ? 0.f : r1 - __uint_as_float(__float_as_uint(r1) & cut2);
     const int gw = col / (GS / 8);  // group within the workgroup slice
-    const uint32_t hi = bf16_rne_bits(ps);
-    uint16_t* sr = sx + row * Tg::SXS + (gw / Tg::NG) * Tg::SXP + gw % Tg::NG;
-    sr[0] = static_cast<uint16_t>(hi);
-    sr[Tg::NGP] = static_cast<uint16_t>(bf16_rne_bits(ps - __uint_as_float(hi << 16)));
+    sx[row * Tg::SXS + (gw / Tg::NG) * Tg::SXP + gw % Tg::NG + spart * Tg::NGP] =
+        static_cast<uint16_t>(__float_as_uint(r) >> 16);
   }
   // zeros in the padding of the group-sum rows (groups NG..NGP of each
-  // half, and past 2 NGP, in every K part)
+  // part, and past 3 NGP, in every K part)
   if (pad)
   for (int e = tid; e < Tg::MR * KH * Tg::SXP; e += Tg::T) {
     const int row = e / (KH * Tg::SXP), t = e % Tg::SXP, part = (e / Tg::SXP) % KH;
-    if (t >= 2 * Tg::NGP || t % Tg::NGP >= Tg::NG) sx[row * Tg::SXS + part * Tg::SXP + t] = 0;
+    if (t >= 3 * Tg::NGP || t % Tg::NGP >= Tg::NG) sx[row * Tg::SXS + part * Tg::SXP + t] = 0;
   }
   __syncthreads();
 }
@@ -381,9 +381,9 @@ __device__ __forceinline__ void tile_accum(f32x4 (&acc)[MT], const TileW<BITS, G
   }
 
   // The bias term sum_g S[m, g] (b[n, g] - OFF s[n, g]) of the wave slice on
-  // the matrix cores: A = the staged group sums (hi and lo halves), B = this
-  // row's biases (and scales) over the same k positions, both halves.  Lane
-  // (r16, gq) supplies k = 32 kb + 8 gq + [0, 8): groups g0.. of one half.
+  // the matrix cores: A = the staged group sums (three parts), B = this row's
+  // biases (and scales) over the same k positions, once per part.  Lane (r16,
+  // gq) supplies k = 32 kb + 8 gq + [0, 8): groups g0.. of one part.
   {
     f32x4 ab[MT], as[MT];
 #pragma unroll
@@ -391,7 +391,7 @@ __device__ __forceinline__ void tile_accum(f32x4 (&acc)[MT], const TileW<BITS, G
 #pragma unroll
     for (int kb = 0; kb < Tg::KB; kb++) {
       const int t0 = 32 * kb + 8 * gq;
-      const bool valid = t0 < 2 * Tg::NGP;
+      const bool valid = t0 < 3 * Tg::NGP;
       const int g0 = t0 % Tg::NGP;
       uint32_t bb[4] = {0u, 0u, 0u, 0u}, bs[4] = {0u, 0u, 0u, 0u};
 #pragma unroll

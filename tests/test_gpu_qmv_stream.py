@@ -109,6 +109,43 @@ def test_stream_and_tile_routes(torch_gpu, monkeypatch, bits, m, n, k, kernel):
     assert rel_err(y[:, rows], orc.qmatmul_f64(x, wq[rows], s[rows], b[rows], 64, bits)) <= TIGHT
 
 
+@pytest.mark.parametrize("bits,m,n,k", [r[:4] for r in ROUTES if "stream" in r[4] or "tile" in r[4]] + [
+    (4, 16, 4096, 4096), (4, 32, 4096, 4096), (8, 16, 1024, 4096), (4, 96, 14336, 4096)])
+def test_group_sums_keep_f32(torch_gpu, monkeypatch, bits, m, n, k):
+    """The affine term's group sums of the activations hold all 24 bits of an
+    f32: every group of a row sums to 189.5, one to 189.5 + 2^-12, and biases
+    of alternating sign (scales of 2^-60, codes 0) cancel all but +-2^-12.  A
+    group sum cut to 16 bits gives 0.  Q8: an infinite activation under
+    weights of one sign gives an infinity in every output of its row."""
+    import torch
+
+    import mlxq
+    for v in ("MLXQ_QMV_TILE_STREAM", "MLXQ_QMV_TILE", "MLXQ_QMV_TILE_ALL"):
+        monkeypatch.delenv(v, raising=False)
+    mlxq.reload_overrides()
+    route = mlxq.qmatmul_route(m, n, k, 64, bits)
+    assert "stream" in route or "tile" in route, route
+    G = k // 64
+    x = torch.full((m, G, 64), 3.0)
+    x[:, :, 0] = 3.5
+    x[:, :, 1] = 0.0
+    hit = (torch.arange(m) * (G - 1) // max(m - 1, 1)).tolist()  # spread over the groups
+    for i, g in enumerate(hit):
+        x[i, g, 1] = 2.0**-12
+    x = x.view(m, k).to(torch.bfloat16).cuda()
+    sign = 1.0 - 2.0 * (torch.arange(G) % 2)
+    wq = torch.zeros((n, k * bits // 32), dtype=torch.int32, device="cuda")
+    s = torch.full((n, G), 2.0**-60, dtype=torch.bfloat16, device="cuda")
+    b = sign.to(torch.bfloat16).cuda().expand(n, G).contiguous()
+    want = (sign[hit] * 2.0**-12 + 189.5 * float(sign.sum()))[:, None].expand(m, n)
+    got = mlxq.qmatmul(x, wq, s, b, 64, bits).float().cpu()
+    assert torch.all((got - want).abs() <= 2.0**-8 * want.abs()), (got[:, 0], want[:, 0])
+    if bits == 8:
+        x[m // 2, k // 2 + 1] = float("inf")
+        got = mlxq.qmatmul(x, wq + 0x01010101, s.fill_(1), s, 64, bits).float()
+        assert torch.isinf(got[m // 2]).all() and torch.isfinite(got[m // 2 + 1:]).all()
+
+
 def test_stream_splits_without_workspace(torch_gpu):
     """Shapes whose default form splits K run on another kernel when the
     workspace has no room for the partials."""
