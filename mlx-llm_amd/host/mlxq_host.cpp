@@ -6,6 +6,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <utility>
 
 #include "mlxq.h"
 
@@ -85,18 +86,19 @@ Array as_bf16(const Array& a) {
   return Array::from_f32(a.to_f32(), a.shape(), DType::BF16);
 }
 
-// qmatmul workspace of the calling device, grown on demand and kept (work
-// queued on the stream may still use an outgrown one until it completes,
-// so the old buffer is retired only after a stream synchronization).
+// qmatmul workspace of the calling device and this thread's stream (calls on
+// different streams can overlap), grown on demand and kept (work queued on
+// the stream may still use an outgrown one until it completes, so the old
+// buffer is retired only after a stream synchronization).
 std::mutex g_ws_mutex;
-std::map<int, Array> g_ws;
+std::map<std::pair<int, hipStream_t>, Array> g_ws;
 
 Array workspace(size_t bytes) {
   if (!bytes) return Array();
   int dev = 0;
   check_hip(hipGetDevice(&dev), "hipGetDevice");
   std::lock_guard<std::mutex> lock(g_ws_mutex);
-  Array& ws = g_ws[dev];
+  Array& ws = g_ws[{dev, g_stream}];
   if (ws.empty() || ws.nbytes() < bytes) {
     if (!ws.empty()) check_hip(hipStreamSynchronize(g_stream), "hipStreamSynchronize");
     ws = Array({static_cast<int64_t>(bytes)}, DType::U8);

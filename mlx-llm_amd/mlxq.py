@@ -208,20 +208,30 @@ def workspace_size(m: int, n: int, k: int, group_size: int = 64, bits: int = 4) 
 
 _ws = {}
 _ws_retired = []
+_ws_lock = threading.Lock()
 
 
 def workspace(nbytes: int, device):
-    """A per-device qmatmul workspace (scratch for split-K partial sums),
-    grown on demand.  A workspace that is outgrown is kept alive, not freed:
-    work already queued or captured in a HIP graph may still use it."""
+    """The qmatmul workspace (scratch for split-K partial sums) of a device's
+    current stream, grown on demand: calls on different streams can overlap,
+    so each stream has its own; calls on one stream, from any thread, run one
+    after the other.  A graph uses the workspace of the stream it was captured
+    on, so graphs of one capture stream must not be replayed at the same time.
+    A workspace that is outgrown is kept alive, not freed: work already queued
+    or captured in a HIP graph may still use it."""
     torch = _torch()
-    key = str(device)
+    dev = torch.device(device)
+    index = torch.cuda.current_device() if dev.index is None and dev.type == "cuda" else dev.index
+    key = (index, _stream())
     cur = _ws.get(key)
     if cur is None or cur.numel() < nbytes:
-        if cur is not None:
-            _ws_retired.append(cur)
-        cur = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-        _ws[key] = cur
+        with _ws_lock:
+            cur = _ws.get(key)
+            if cur is None or cur.numel() < nbytes:
+                if cur is not None:
+                    _ws_retired.append(cur)
+                cur = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=dev)
+                _ws[key] = cur
     return cur
 
 
@@ -264,7 +274,8 @@ def bind_qmatmul(x, wq, scales, biases, group_size: int = 64, bits: int = 4, out
                  algo: int = ALGO_AUTO):
     """Pre-resolve every pointer of one qmatmul call and return a zero-argument
     callable that launches it on the then-current stream (for tight loops and
-    HIP-graph capture; the workspace is allocated here, never in the call)."""
+    HIP-graph capture; the current stream's workspace is allocated here, that
+    of another stream in the first call on it)."""
     torch = _torch()
     k = x.shape[-1]
     n = wq.shape[0]
@@ -273,11 +284,16 @@ def bind_qmatmul(x, wq, scales, biases, group_size: int = 64, bits: int = 4, out
     nbytes = workspace_size(m, n, k, group_size, bits)
     ws = workspace(nbytes, x.device) if nbytes else None
     f = lib().mlxq_qmatmul_algo
-    args = (_ptr(x), m, _ptr(wq), _ptr(scales), _ptr(biases), _ptr(bias), n, k, group_size, bits, _ptr(y),
-            _ptr(ws), 0 if ws is None else ws.numel(), algo)
+    args = (_ptr(x), m, _ptr(wq), _ptr(scales), _ptr(biases), _ptr(bias), n, k, group_size, bits, _ptr(y))
+    own = (*args, _ptr(ws), 0 if ws is None else ws.numel(), algo)
+    device, bound = x.device, _stream()
 
     def call():
-        rc = f(*args, _stream())
+        st = _stream()
+        if ws is None or st == bound:
+            rc = f(*own, st)
+        else:
+            rc = f(*args, workspace(ws.numel(), device).data_ptr(), ws.numel(), algo, st)
         if rc:
             check(rc)
         return y

@@ -133,7 +133,8 @@ class DecodeStack:
         self.d = e(cfg.hidden)
         self.logits = e(cfg.vocab)
         # the qmatmul workspace for the largest projection call of any batch
-        # <= batch, reserved now so that no call grows it inside a capture
+        # <= batch, reserved now so that no call on this stream grows it
+        # (capture() warms up the workspace of its own stream)
         shapes = [(p.n, p.k) for p in [*self.layers[0].proj.values(), self.lm_head]]
         need = max(mlxq.workspace_size(b, n, k, cfg.group_size, cfg.bits)
                    for b in range(1, batch + 1) for n, k in shapes)

@@ -118,6 +118,32 @@ def test_workspace_sizes_cover_every_decode_shape():
                 mlxq.workspace_size(m, n, k, 64, bits)
 
 
+def test_workspace_per_stream(monkeypatch):
+    """Calls on two streams never share scratch; one stream keeps its buffer,
+    also from another thread, until a larger one is asked for, and the
+    outgrown one stays alive."""
+    import threading
+
+    stream = [1]
+    monkeypatch.setattr(mlxq, "_stream", lambda: stream[0])
+    monkeypatch.setattr(mlxq, "_ws", {})
+    monkeypatch.setattr(mlxq, "_ws_retired", [])
+    a = mlxq.workspace(1 << 20, "cpu")
+    got = []
+    t = threading.Thread(target=lambda: got.append(mlxq.workspace(1000, "cpu")))
+    t.start()
+    t.join()
+    assert got[0] is a
+    stream[0] = 2
+    b = mlxq.workspace(1 << 20, "cpu")
+    assert b.data_ptr() != a.data_ptr()
+    big = mlxq.workspace(1 << 21, "cpu")
+    assert big.numel() >= 1 << 21 and big.data_ptr() not in (a.data_ptr(), b.data_ptr())
+    assert mlxq._ws_retired[0] is b
+    stream[0] = 1
+    assert mlxq.workspace(1 << 20, "cpu") is a
+
+
 def test_header_compiles_as_c99(tmp_path):
     """include/mlxq.h is a plain C header (the boundary binds from C / cgo /
     bindgen): it compiles alone under -std=c99 -pedantic with warnings as errors."""

@@ -555,3 +555,37 @@ def test_calls_follow_the_current_stream(torch_gpu, monkeypatch):
     monkeypatch.delenv("MLXQ_QMV_STREAM64")
     mlxq.reload_overrides()
     assert size() == before
+
+
+@pytest.mark.parametrize("m,n,k", [(8, 5120, 5120), (118, 2048, 5632)])
+def test_split_k_calls_on_two_streams(torch_gpu, m, n, k):
+    """Calls that split K, queued on two streams that overlap: each keeps its
+    partial sums in its own stream's workspace, so every result is that of
+    the call alone; a bound call takes the workspace of the stream it runs on."""
+    import torch
+
+    assert "split_reduce" in mlxq.qmatmul_route(m, n, k, 64, 4)
+    wq, s, b = make_layer(0x2A + k, n, k, 64, 4)
+    w = dev(wq), dev(s, bf16=True), dev(b, bf16=True)
+    xs = [dev(bf16_acts(0x2B + i, m, k), bf16=True) for i in range(2)]
+    want = [mlxq.qmatmul(x, *w, 64, 4) for x in xs]
+    bound = mlxq.bind_qmatmul(xs[1], *w, 64, 4)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in xs]
+    ptrs, got = set(), [[], []]
+    for _ in range(20):
+        for i, st in enumerate(streams):
+            with torch.cuda.stream(st):
+                got[i].append(mlxq.qmatmul(xs[i], *w, 64, 4))
+                ptrs.add(mlxq.workspace(1, xs[i].device).data_ptr())
+    torch.cuda.synchronize()
+    assert len(ptrs) == 2 and mlxq.workspace(1, xs[0].device).data_ptr() not in ptrs
+    for i in range(2):
+        assert all(torch.equal(y, want[i]) for y in got[i]), i
+    for _ in range(20):
+        with torch.cuda.stream(streams[0]):
+            y = mlxq.qmatmul(xs[0], *w, 64, 4)
+        with torch.cuda.stream(streams[1]):
+            bound()
+    torch.cuda.synchronize()
+    assert torch.equal(y, want[0]) and torch.equal(bound.out, want[1])
