@@ -18,10 +18,13 @@ namespace mlxq {
 namespace {  // internal linkage: each including file has its own copy
 
 // Correctly rounded x / n for finite x of ordinary magnitude (the quotient's
-// residual is then exact): the quotient estimate and one residual step.  With
-// n = 15 or 255 and r = RN(1/n), and with n = 1 .. 257 and r = v_rcp_f32(n),
-// this equals the f32 division for every mantissa of x (checked over all 2^23
-// of them on gfx950); the compiler's general division is 11 instructions.
+// residual is then exact): the quotient estimate and one residual step.  For
+// n = 1 .. 257 and r within one ulp of 1/n (v_rcp_f32, and RN(1/n) for the
+// constants 15 and 255) this equals the f32 division for every mantissa of x
+// (tests/cpp/quotient_sweep.cpp); the compiler's general division is 11
+// instructions.  Larger n can be off by an ulp: with x = 0x1.b5b6b2p-1 and n =
+// x / 1e-7, a constant group, one of the reciprocals within an ulp of 1/n
+// gives another quotient.
 __device__ __forceinline__ float div_by(float x, float n, float r) {
   const float q = x * r;
   return fmaf(fmaf(-n, q, x), r, q);
@@ -83,10 +86,12 @@ __device__ __forceinline__ void quantize_group(const float (&v)[EPL], uint32_t (
   // fma(x, r1, x r2) with r1 + r2 = 1/s to about 48 bits: the two quotients
   // can only round apart next to a half-integer, and there they were compared
   // on gfx950 for every mantissa of s, every half-integer up to 256.5 and the
-  // nine x around their product; the one mantissa that differs (all ones,
-  // x/s next to 0.5) takes the division below.  The comparison carries over
-  // to any scale whose products neither overflow nor lose their residuals: s
-  // is at least 1e-7, and |x| at most 2^60 is tested.
+  // nine x around their product (on the CPU, with every reciprocal within an
+  // ulp and most of those mantissas: tests/cpp/quotient_sweep.cpp); the one
+  // mantissa that differs (all ones, x/s next to 0.5) takes the division
+  // below.  The comparison carries over to any scale whose products neither
+  // overflow nor lose their residuals: s is at least 0.5e-7, and |x| at most
+  // 2^60 is tested.
   auto recip = [](float s, float& r1, float& r2) {
     const float r0 = __builtin_amdgcn_rcpf(s);
     r1 = fmaf(fmaf(-s, r0, 1.0f), r0, r0);
@@ -97,12 +102,16 @@ __device__ __forceinline__ void quantize_group(const float (&v)[EPL], uint32_t (
   const float q0 = __builtin_rintf(fmaf(edge, r1, edge * r2));
   bias = 0.f;
   if (q0 != 0.f) {
-    scale = div_by(edge, q0, __builtin_amdgcn_rcpf(q0));  // |q0| <= n_bins + 1
+    scale = div_by(edge, q0, __builtin_amdgcn_rcpf(q0));
     bias = edge;
   }
   recip(scale, r1, r2);
-  // false for an infinite or NaN edge too (a finite edge bounds the group)
-  const bool ordinary = fabsf(edge) <= 0x1p60f && (__float_as_uint(scale) & 0x7FFFFFu) != 0x7FFFFFu;
+  // false for an infinite or NaN edge too (a finite edge bounds the group).
+  // |q0| is at most n_bins + 1 in a group with values of both signs, but edge
+  // / scale, up to 2^60 / 1e-7, in a narrow one of one sign: past 256 neither
+  // quotient above was compared.
+  const bool ordinary = fabsf(edge) <= 0x1p60f && fabsf(q0) <= 256.f &&
+                        (__float_as_uint(scale) & 0x7FFFFFu) != 0x7FFFFFu;
   // The quotient lies in [0, n_bins + 1] (bias is the group's edge and scale
   // of the sign that makes it positive; with bias 0 it rounds to 0); a NaN
   // element clamps to 0.  Adding 2^23 rounds it to the nearest integer, ties

@@ -156,6 +156,31 @@ def test_groups_outside_the_ordinary_range(torch_gpu, bits, gs, bf16):
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("gs", [32, 64, 128])
 @pytest.mark.parametrize("bf16", [True, False])
+def test_narrow_groups_of_one_sign(torch_gpu, bits, gs, bf16):
+    """Groups whose values have one sign and a small spread: edge / scale runs
+    from the number of bins to 2^30 (constant groups: scale 1e-7), far past
+    the quotients of a group around zero.  The first values are the constant
+    groups for which a reciprocal one ulp off changes the last bit of the
+    scale.  Codes, scales and biases bit-exact."""
+    rng = np.random.default_rng(0x51 + gs)
+    hard = [float.fromhex("0x1.b5b6b2p-1") * 2.0**e for e in range(12)]
+    level = np.float32(hard + list(np.exp(rng.uniform(np.log(1e-3), np.log(1e3), 500))))
+    spread = np.where(np.arange(512) % 4 == 0, 0.0, np.exp(rng.uniform(np.log(1e-7), np.log(0.9), 512)))
+    spread[:len(hard)] = 0
+    sign = np.where(np.arange(512) % 2, -1.0, 1.0)
+    w = level[:, None] * (1.0 - spread[:, None] * rng.random((512, gs))) * sign[:, None]
+    w = w.astype(np.float32).reshape(128, 4 * gs)
+    if bf16:
+        w = orc.f32_to_bf16(w).reshape(128, 4 * gs)
+    ref = orc.affine_quantize(w, gs, bits, orc.BF16 if bf16 else orc.F32)
+    got = gpu_quantize(w, gs, bits, bf16)
+    for r, g in zip(ref, got):
+        assert np.array_equal(np.asarray(r).view(np.uint8), np.asarray(g).view(np.uint8))
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("bf16", [True, False])
 @pytest.mark.parametrize("rows,cols", [(1, 128), (3, 384), (33, 640)])
 def test_dequantize_partial_workgroups(torch_gpu, bits, gs, bf16, rows, cols):
     import torch

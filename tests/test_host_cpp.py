@@ -75,3 +75,19 @@ def test_safetensors_interop(tmp_path):
     for k, v in src.items():
         assert back[k].dtype == v.dtype and back[k].shape == v.shape, k
         assert torch.equal(back[k].view(torch.uint8), v.view(torch.uint8)), k
+
+
+def test_quantizer_quotient_sweep(tmp_path):
+    """The two short quotients of the affine quantizer equal the f32 division
+    over every mantissa they are used for, with any reciprocal estimate
+    within one ulp (tests/cpp/quotient_sweep.cpp)."""
+    import shutil
+
+    if not shutil.which("g++") or " fma " not in Path("/proc/cpuinfo").read_text():
+        pytest.skip("needs g++ and a CPU with FMA")
+    src = Path(__file__).parent / "cpp" / "quotient_sweep.cpp"
+    exe = tmp_path / "quotient_sweep"
+    subprocess.run(["g++", "-O3", "-std=c++17", "-march=native", "-ffp-contract=off", "-fno-math-errno",
+                    "-fno-trapping-math", "-pthread", str(src), "-o", str(exe)], check=True, timeout=120)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
