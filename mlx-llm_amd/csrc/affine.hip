@@ -19,7 +19,10 @@ namespace {
 
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+// code words: any 4-byte alignment (one instruction each all the same)
+typedef u32x2 u32x2_words __attribute__((aligned(4)));
+typedef u32x4 u32x4_words __attribute__((aligned(4)));
 
 constexpr int kThreads = 256;
 
@@ -72,8 +75,8 @@ __global__ __launch_bounds__(kThreads) void affine_quantize_kernel(const void* _
   quantize_group<BITS, LPG, EPL>(v, words, scale, bias);  // n_lanes is a multiple of LPG: a group's lanes are all real or all clamped
   if (lane >= n_lanes) return;
   if constexpr (W == 1) wq[lane] = words[0];
-  else if constexpr (W == 2) reinterpret_cast<uint2*>(wq)[lane] = make_uint2(words[0], words[1]);
-  else reinterpret_cast<uint4*>(wq)[lane] = make_uint4(words[0], words[1], words[2], words[3]);
+  else if constexpr (W == 2) *reinterpret_cast<u32x2_words*>(wq + lane * W) = u32x2{words[0], words[1]};
+  else *reinterpret_cast<u32x4_words*>(wq + lane * W) = u32x4{words[0], words[1], words[2], words[3]};
   if ((threadIdx.x & (LPG - 1)) == 0) {
     const int64_t g = lane / LPG;
     store1<DT>(scales, g, scale);

@@ -65,8 +65,9 @@ __device__ __forceinline__ void round_bf16(float (&v)[N]) {
   }
 }
 
-// the words of a lane's codes (16-byte stores), and its group's scale and
-// bias from the group's first lane
+// the words of a lane's codes (16-byte stores, wq at any 8-byte alignment),
+// and its group's scale and bias from the group's first lane
+typedef uint32_t u32x4_words __attribute__((ext_vector_type(4), aligned(8)));
 template <int BITS, int LPG, int EPL>
 __device__ __forceinline__ void store_group(const uint32_t (&words)[EPL * BITS / 32], float scale, float bias,
                                             int64_t lane, uint32_t* wq, uint16_t* scales, uint16_t* biases) {
@@ -76,8 +77,8 @@ __device__ __forceinline__ void store_group(const uint32_t (&words)[EPL * BITS /
   } else {
 #pragma unroll
     for (int j = 0; j < W / 4; j++)
-      reinterpret_cast<uint4*>(wq)[lane * (W / 4) + j] =
-          make_uint4(words[4 * j], words[4 * j + 1], words[4 * j + 2], words[4 * j + 3]);
+      *reinterpret_cast<u32x4_words*>(wq + lane * W + 4 * j) =
+          u32x4_words{words[4 * j], words[4 * j + 1], words[4 * j + 2], words[4 * j + 3]};
   }
   if ((threadIdx.x & (LPG - 1)) == 0) {
     const int64_t g = lane / LPG;

@@ -194,3 +194,29 @@ def test_dequantize_partial_workgroups(torch_gpu, bits, gs, bf16, rows, cols):
     got = mlxq.dequantize(dev(wq), dev(s, bf16=bf16), dev(b, bf16=bf16), gs, bits)
     torch.cuda.synchronize()
     assert np.array_equal(host(got).view(np.uint8), np.asarray(ref).view(np.uint8))
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("bf16", [True, False])
+def test_quantize_codes_at_word_alignment(torch_gpu, bits, bf16):
+    """The code words may start at any 4-byte (Q8: 8-byte) boundary, although
+    a lane stores up to four of them at once: bit-exact, and nothing before or
+    after the array is written."""
+    import torch
+
+    n, k, gs = 33, 640, 64
+    w = bf16_weights(0x61 + bits, n, k)
+    if not bf16:
+        w = orc.normal(0x62 + bits, n * k, 0.0, 0.02).reshape(n, k)
+    ref = orc.affine_quantize(w, gs, bits, orc.BF16 if bf16 else orc.F32)
+    words, step = n * k * bits // 32, bits // 4
+    for off in range(step, 5, step):
+        buf = torch.full((words + 8,), -1, dtype=torch.int32, device="cuda")
+        x = dev(w, bf16=bf16)
+        s = torch.empty((n, k // gs), dtype=x.dtype, device="cuda")
+        b = torch.empty_like(s)
+        mlxq.check(mlxq.lib().mlxq_quantize(x.data_ptr(), mlxq.BF16 if bf16 else mlxq.F32, n, k, gs, bits,
+                                            buf.data_ptr() + 4 * off, s.data_ptr(), b.data_ptr(), mlxq._stream()))
+        got = host(buf)
+        assert np.array_equal(got[off:off + words], ref[0].reshape(-1).view(np.uint32)), off
+        assert np.all(got[:off] == 0xFFFFFFFF) and np.all(got[off + words:] == 0xFFFFFFFF)

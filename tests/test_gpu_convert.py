@@ -79,6 +79,26 @@ def test_requantize_llama3_shapes(torch_gpu, name, rows, cols, heads):
         assert np.array_equal(g, w)
 
 
+@pytest.mark.parametrize("name", ["Q4_0", "Q6_K", "BF16", "F32"])
+@pytest.mark.parametrize("bits", [4, 8])
+def test_requantize_codes_at_8_byte_alignment(torch_gpu, name, bits):
+    """The code words may start at any 8-byte boundary, although a lane stores
+    16 bytes at once: bit-exact, and nothing before or after is written."""
+    import torch
+
+    tag, rows, cols = TAGS[name], 33, 768
+    data = blocks(tag, rows, cols, 930 + tag)
+    want = orc.gguf_requantize(tag, data, rows, cols, 0, 64, bits)
+    words = rows * cols * bits // 32
+    buf = torch.full((words + 8,), -1, dtype=torch.int32, device="cuda")
+    s = torch.empty((rows, cols // 64), dtype=torch.bfloat16, device="cuda")
+    b = torch.empty_like(s)
+    mlxq.gguf_requantize(tag, torch.from_numpy(data).cuda(), rows, cols, 0, 64, bits, out=(buf[2:], s, b))
+    got = host(buf)
+    assert np.array_equal(got[2:2 + words], np.asarray(want[0]).reshape(-1).view(np.uint32))
+    assert np.all(got[:2] == 0xFFFFFFFF) and np.all(got[2 + words:] == 0xFFFFFFFF)
+
+
 def test_requantize_errors(torch_gpu):
     import torch
 
