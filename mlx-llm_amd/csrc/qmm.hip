@@ -147,7 +147,8 @@ struct QmmGeom {
 // Two requests for consecutive KB of LDS: the instruction's offset moves the
 // LDS destination and the memory address alike, so one M0 serves both, and
 // off1 is the second request's offset less 1024 (from a base 1024 lower, so
-// that it cannot be negative).
+// that it cannot be negative).  Every first offset is then 1024 more than the
+// byte it names and has to fit 32 bits all the same.
 constexpr uint32_t kDmaBias = 1024;
 __device__ __forceinline__ void dma16x2_to_lds_sbase(const void* base, uint32_t off0, uint32_t off1,
                                                      unsigned char* lds) {
@@ -231,19 +232,26 @@ __global__ __launch_bounds__(256, 1) void qmm_kernel(const uint16_t* __restrict_
   const uint32_t row_bytes = static_cast<uint32_t>(K) * BITS / 8;
 
   // ---- DMA sources: per-lane byte offsets (32-bit: the host checks sizes)
-  // activations: 1 KB chunk q = 8 rows; lane -> row 8q + lane/8, chunk position lane % 8
+  // activations: 1 KB chunk q = 8 rows; lane -> row 8q + lane/8, chunk position
+  // lane % 8 (at most M K 2 + 112, K a multiple of 512: it fits wherever the
+  // activations are below 4 GiB)
   uint32_t a_off[Gm::A_DMA];
 #pragma unroll
   for (int i = 0; i < Gm::A_DMA; i++) {
     const int r = 8 * (wave * Gm::A_DMA + i) + (lane >> 3), c = (lane & 7) ^ swz(r);
     a_off[i] = (static_cast<uint32_t>(min(m0 + r, M - 1)) * K + kb + 8 * c) * 2 + (i & 1 ? 0 : kDmaBias);
   }
-  // codes: the same row / chunk mapping over 128-byte code lines
+  // codes: the same row / chunk mapping over 128-byte code lines.  From nine
+  // rows of weights on, a second request's row is at least row 8, and no base
+  // has to be lowered: codes of up to 4 GiB, whose last rows have no room for
+  // a larger offset.
+  const uint32_t code_bias = N > 8 ? 0 : kDmaBias;
   uint32_t c_off[Gm::C_DMA];
 #pragma unroll
   for (int i = 0; i < Gm::C_DMA; i++) {
     const int r = 8 * (wave * Gm::C_DMA + i) + (lane >> 3), c = (lane & 7) ^ swz(r);
-    c_off[i] = static_cast<uint32_t>(min(n0 + r, N - 1)) * row_bytes + kb * BITS / 8 + 16 * c + (i & 1 ? 0 : kDmaBias);
+    c_off[i] = static_cast<uint32_t>(min(n0 + r, N - 1)) * row_bytes + kb * BITS / 8 + 16 * c +
+               (i & 1 ? code_bias - kDmaBias : code_bias);
   }
   // scales / biases: per row [scales SROW bytes][biases SROW bytes]; lanes
   // (row, array, 16-byte part)
@@ -259,13 +267,13 @@ __global__ __launch_bounds__(256, 1) void qmm_kernel(const uint16_t* __restrict_
 
   // DMA of the activations of step kt / code batch c / scale batch sb into
   // stage / buffer `buf` (the index is clamped past the end, the buffer not)
-  // pair i of this wave's share of a DMA (the offsets carry kDmaBias)
+  // pair i of this wave's share of a DMA (the offsets carry the bias)
   auto dma_a1 = [&](int kt, int buf, int i) __attribute__((always_inline)) {
     dma16x2_to_lds_sbase(reinterpret_cast<const char*>(x) + kt * (BK * 2) - kDmaBias, a_off[2 * i], a_off[2 * i + 1],
                          lds + Gm::A_OFF + buf * Gm::A_BYTES + (wave * Gm::A_DMA + 2 * i) * 1024);
   };
   auto dma_c1 = [&](int c, int buf, int i) __attribute__((always_inline)) {  // steps CB c .. CB c + CB - 1
-    dma16x2_to_lds_sbase(reinterpret_cast<const char*>(wq) + c * 128 - kDmaBias, c_off[2 * i], c_off[2 * i + 1],
+    dma16x2_to_lds_sbase(reinterpret_cast<const char*>(wq) + c * 128 - code_bias, c_off[2 * i], c_off[2 * i + 1],
                          lds + Gm::C_OFF + buf * Gm::C_BYTES + (wave * Gm::C_DMA + 2 * i) * 1024);
   };
   auto dma_s1 = [&](int sb, int buf, int i) __attribute__((always_inline)) {  // steps 8 sb .. 8 sb + 7
@@ -754,7 +762,7 @@ int launch_qmm(const uint16_t* x, int64_t M, const uint32_t* wq, const uint16_t*
                const uint16_t* bias, int64_t N, int64_t K, int group_size, int bits, uint16_t* y, void* workspace,
                size_t workspace_bytes, hipStream_t st) {
   // the DMA offsets are 32-bit byte offsets from the array bases
-  if (M * K * 2 + kDmaBias >= (int64_t(1) << 32) || N * K * bits / 8 + kDmaBias >= (int64_t(1) << 32) || !qmm_eligible(K, group_size))
+  if (M * K * 2 >= (int64_t(1) << 32) || N * K * bits / 8 >= (int64_t(1) << 32) || !qmm_eligible(K, group_size))
     return fail(MLXQ_ERR_UNSUPPORTED, "qmm: activations and codes must each be below 4 GiB, K a multiple of " +
                                           std::to_string(PERIOD * BK) + " and of 8 groups");
   const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);

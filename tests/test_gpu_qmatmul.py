@@ -528,6 +528,35 @@ def test_route_query_names_the_kernels(torch_gpu):
     assert r(512, 4096, 4096, 64, 4, workspace_bytes=0) == "qmm_kernel<4, 64, 4, 2>"  # no workspace: unsplit
 
 
+@pytest.mark.parametrize("bits,m,n,k", [(4, 40, 5592405, 1536), (8, 40, 8388607, 512), (4, 1398101, 72, 1536),
+                                        (4, 40, 5, 512), (8, 33, 9, 512)])
+def test_qmm_operands_just_below_4_gib(torch_gpu, bits, m, n, k):
+    """The prefill kernel's 32-bit offsets reach the last rows of codes and
+    activations of up to 256 (1024) bytes below 4 GiB, and the rows of
+    matrices of a few rows: the first and last rows of both against the f64
+    product of the dequantized rows."""
+    import torch
+
+    g = torch.Generator("cuda").manual_seed(0x4600 + n)
+    wq = torch.randint(-2**31, 2**31, (n, k * bits // 32), dtype=torch.int32, device="cuda", generator=g)
+    s = torch.rand((n, k // 64), dtype=torch.bfloat16, device="cuda", generator=g) * 0.01 + 0.001
+    b = s * -(2.0 ** (bits - 1))
+    x = torch.randn((m, k), dtype=torch.bfloat16, device="cuda", generator=g)
+    assert m * k * 2 < 2**32 and n * k * bits // 8 < 2**32
+    y = mlxq.qmatmul(x, wq, s, b, 64, bits, algo=mlxq.ALGO_QMM)
+    rows = sorted({*range(min(n, 300)), *range(max(0, n - 300), n)})
+    acts = sorted({*range(min(m, 300)), *range(max(0, m - 300), m)})
+    w = mlxq.dequantize(wq[rows].contiguous(), s[rows].contiguous(), b[rows].contiguous(), 64, bits)
+    ref = x[acts].double() @ w.double().T
+    got = y[acts][:, rows].double()
+    assert rel_err(got.cpu().numpy(), ref.cpu().numpy()) <= TIGHT
+    # and, spread over the whole operands, rows between them
+    rows = torch.arange(0, n, max(1, n // 500), device="cuda")
+    w = mlxq.dequantize(wq[rows], s[rows], b[rows], 64, bits)
+    ref = x[acts].double() @ w.double().T
+    assert rel_err(y[acts][:, rows].double().cpu().numpy(), ref.cpu().numpy()) <= TIGHT
+
+
 def test_calls_follow_the_current_stream(torch_gpu, monkeypatch):
     """The raw stream handle that calls launch on is torch's current one: the
     default stream, a side stream, and each thread's own; workspace_size()
