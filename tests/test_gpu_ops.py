@@ -106,6 +106,9 @@ def test_ops_reject_bad_shapes(torch_gpu):
     (4, 24, 4096, 4096, False),   # one K slice: the projection, then add and norm
     (4, 2, 14336, 4096, False),   # batch 2: the unfused calls
     (8, 40, 2048, 1024, True),    # prefill rows
+    (4, 8, 11008, 4096, True),    # eight uneven splits of 43 slices
+    (4, 17, 13824, 5120, False),  # of 54 slices, 32 rows per workgroup
+    (8, 32, 5632, 2048, False),   # of 22 slices
 ])
 def test_qmatmul_add_rms_norm(torch_gpu, bits, m, k, n, with_bias):
     """Down projection + residual + next norm (llama.rs:729-733, :698) in one

@@ -92,8 +92,8 @@ ROUTES = [
 @pytest.mark.parametrize("bits,m,n,k,kernel", ROUTES)
 def test_stream_and_tile_routes(torch_gpu, monkeypatch, bits, m, n, k, kernel):
     """Both sides of each line of the default dispatch of batched decode away
-    from the Llama-3-8B shapes: the kernel's name, and (up to 2^25 codes; the
-    larger shapes run the same forms) sampled rows against the oracle."""
+    from the Llama-3-8B shapes: the kernel's name, and sampled rows against
+    the oracle (above 2^25 codes: random codes, scales and biases)."""
     import mlxq
     for v in ("MLXQ_QMV_TILE_STREAM", "MLXQ_QMV_TILE", "MLXQ_QMV_TILE_ALL"):
         monkeypatch.delenv(v, raising=False)
@@ -101,8 +101,12 @@ def test_stream_and_tile_routes(torch_gpu, monkeypatch, bits, m, n, k, kernel):
     assert kernel in mlxq.qmatmul_route(m, n, k, 64, bits).replace(" ", "").replace("_kernel<", "<").replace(
         "qmv<", "qmv_kernel<")
     if n * k > 1 << 25:
-        return
-    wq, s, b = make_layer(0x120 + bits, n, k, 64, bits)
+        rng = np.random.default_rng(0x120 + bits)
+        wq = rng.integers(0, 1 << 32, (n, k * bits // 32), dtype=np.uint32)
+        s = orc.f32_to_bf16(rng.uniform(0.001, 0.01, (n, k // 64)).astype(np.float32)).reshape(n, -1)
+        b = orc.f32_to_bf16(-(orc.bf16_to_f32(s).reshape(n, -1) * 2.0 ** (bits - 1)).astype(np.float32)).reshape(n, -1)
+    else:
+        wq, s, b = make_layer(0x120 + bits, n, k, 64, bits)
     x = bf16_acts(0x121 + m, m, k)
     y = run(x, wq, s, b, 64, bits)
     rows = np.unique(np.concatenate([np.random.default_rng(0x122).choice(n, 128, replace=False), np.arange(n - 16, n)]))
