@@ -896,10 +896,15 @@ int run_stream(const TileParams& a, int tiles, int mblocks, hipStream_t st) {
   return check_launch("qmv_stream");
 }
 
+// queried once: the dispatch rules below ask for it up to four times per call
 int cu_count() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) return 256;
+  static const int cus = [] {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+      return 256;
+    return n;
+  }();
   return cus;
 }
 
