@@ -15,7 +15,8 @@
 //    VALU), in whole 128-byte lines: the memory path pays per line touched,
 //    so a 32-byte slice of a code row costs as much as a full line.
 //      - activations: the BM x 64 bf16 tile of one step (one line per row),
-//        four stages (128-row tiles) or two, requested that many steps ahead;
+//        four stages (128-row tiles; short Q8 slices of group size 32 two) or
+//        two, requested that many steps ahead;
 //      - codes: 128 bytes of each of the 256 weight rows (4 steps at Q4, 2
 //        at Q8), two buffers, requested a few at a time over the steps;
 //      - scales and biases: 16 bytes per row and array (8 steps of groups),
@@ -64,7 +65,7 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 constexpr int BK = 64;      // K per step
 constexpr int PERIOD = 8;   // steps per unrolled period (one scale batch)
 
-template <int BITS, int GS, int TM, int TN>
+template <int BITS, int GS, int TM, int TN, int ST>
 struct QmmGeom {
   static constexpr int WAVES = 4, THREADS = 64 * WAVES;
   static constexpr int BN = 256;               // weight rows per workgroup
@@ -77,7 +78,7 @@ struct QmmGeom {
   static constexpr int C_BYTES = BN * 128;
   static constexpr int SROW = GS == 32 ? 32 : 16;  // scale bytes per row per batch (and bias bytes)
   static constexpr int S_BYTES = BN * 2 * SROW;
-  static constexpr int AST = TM <= 4 ? 4 : 2;  // activation stages: as many as fit
+  static constexpr int AST = ST;  // activation stages
   static constexpr int A_OFF = 0, C_OFF = AST * A_BYTES, S_OFF = C_OFF + 2 * C_BYTES;
   static constexpr int LDS_BYTES = S_OFF + 2 * S_BYTES;
   // DMA instructions per wave: activations per step, codes / scales per batch
@@ -202,15 +203,13 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
-template <int BITS, int GS, int TM, int TN>
-__global__ __launch_bounds__(256, 1) void qmm_kernel(const uint16_t* __restrict__ x, int M,
-                                                     const uint32_t* __restrict__ wq,
-                                                     const uint16_t* __restrict__ scales,
-                                                     const uint16_t* __restrict__ biases,
-                                                     const uint16_t* __restrict__ bias_vec, int N, int K,
-                                                     uint16_t* __restrict__ y, float* __restrict__ part, int grain,
-                                                     int slice_grains, int longer) {
-  using Gm = QmmGeom<BITS, GS, TM, TN>;
+template <int BITS, int GS, int TM, int TN, int ST>
+__device__ __forceinline__ void qmm_tile(const uint16_t* __restrict__ x, int M, const uint32_t* __restrict__ wq,
+                                         const uint16_t* __restrict__ scales, const uint16_t* __restrict__ biases,
+                                         const uint16_t* __restrict__ bias_vec, int N, int K,
+                                         uint16_t* __restrict__ y, float* __restrict__ part, int grain,
+                                         int slice_grains, int longer) {
+  using Gm = QmmGeom<BITS, GS, TM, TN, ST>;
   constexpr int BM = Gm::BM, BN = Gm::BN, CB = Gm::CB;
   extern __shared__ __align__(16) unsigned char lds[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -686,11 +685,37 @@ __global__ __launch_bounds__(256, 1) void qmm_kernel(const uint16_t* __restrict_
   }
 }
 
+// As many activation stages as fit; two for short slices (see launch_cfg).
 template <int BITS, int GS, int TM, int TN>
+__global__ __launch_bounds__(256, 1) void qmm_kernel(const uint16_t* __restrict__ x, int M,
+                                                     const uint32_t* __restrict__ wq,
+                                                     const uint16_t* __restrict__ scales,
+                                                     const uint16_t* __restrict__ biases,
+                                                     const uint16_t* __restrict__ bias_vec, int N, int K,
+                                                     uint16_t* __restrict__ y, float* __restrict__ part, int grain,
+                                                     int slice_grains, int longer) {
+  qmm_tile<BITS, GS, TM, TN, TM <= 4 ? 4 : 2>(x, M, wq, scales, biases, bias_vec, N, K, y, part, grain, slice_grains,
+                                              longer);
+}
+template <int BITS, int GS, int TM, int TN>
+__global__ __launch_bounds__(256, 1) void qmm_short_kernel(const uint16_t* __restrict__ x, int M,
+                                                           const uint32_t* __restrict__ wq,
+                                                           const uint16_t* __restrict__ scales,
+                                                           const uint16_t* __restrict__ biases,
+                                                           const uint16_t* __restrict__ bias_vec, int N, int K,
+                                                           uint16_t* __restrict__ y, float* __restrict__ part,
+                                                           int grain, int slice_grains, int longer) {
+  qmm_tile<BITS, GS, TM, TN, 2>(x, M, wq, scales, biases, bias_vec, N, K, y, part, grain, slice_grains, longer);
+}
+
+template <int BITS, int GS, int TM, int TN, bool SHORT = false>
 int launch(const uint16_t* x, int M, const uint32_t* wq, const uint16_t* s, const uint16_t* b, const uint16_t* bias,
            int N, int K, uint16_t* y, float* part, int splits, hipStream_t st) {
-  using Gm = QmmGeom<BITS, GS, TM, TN>;
-  auto kern = qmm_kernel<BITS, GS, TM, TN>;
+  using Gm = QmmGeom<BITS, GS, TM, TN, (SHORT || TM > 4) ? 2 : 4>;
+  auto kern = [] {
+    if constexpr (SHORT) return &qmm_short_kernel<BITS, GS, TM, TN>;
+    else return &qmm_kernel<BITS, GS, TM, TN>;
+  }();
   static bool attr_set = false;  // once per process; the attribute is per function
   if (!attr_set) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -733,7 +758,18 @@ int qmm_cfg(int64_t M, int64_t N, int splits) {
 template <int BITS, int GS>
 int launch_cfg(const uint16_t* x, int M, const uint32_t* wq, const uint16_t* s, const uint16_t* b, const uint16_t* bias,
                int N, int K, uint16_t* y, float* part, int splits, hipStream_t st) {
-  if (qmm_cfg(M, N, splits) == 42) return launch<BITS, GS, 4, 2>(x, M, wq, s, b, bias, N, K, y, part, splits, st);
+  if (qmm_cfg(M, N, splits) == 42) {
+    // Q8 of group size 32 has the most bytes per step, and slices of up to 16
+    // steps end before the deeper prefetch pays for what it requests past
+    // their end: two activation stages (us with four / two; K steps per slice
+    // in brackets): 300 x 1024 x 1024 (8) 17.6 / 16.7, 64 x 17408 x 1024 (16)
+    // 19.6 / 19.4, 300 x 4096 x 4096 (16) 29.7 / 29.5, 300 x 4096 x 6144 (24)
+    // 36.5 / 36.8, 333 x 4096 x 14336 (48) 67.3 / 70.0.
+    if constexpr (BITS == 8 && GS == 32)
+      if (ceil_div(K / (PERIOD * BK), splits) <= 2)
+        return launch<BITS, GS, 4, 2, true>(x, M, wq, s, b, bias, N, K, y, part, splits, st);
+    return launch<BITS, GS, 4, 2>(x, M, wq, s, b, bias, N, K, y, part, splits, st);
+  }
   return launch<BITS, GS, 8, 2>(x, M, wq, s, b, bias, N, K, y, part, splits, st);
 }
 

@@ -528,6 +528,23 @@ def test_route_query_names_the_kernels(torch_gpu):
     assert r(512, 4096, 4096, 64, 4, workspace_bytes=0) == "qmm_kernel<4, 64, 4, 2>"  # no workspace: unsplit
 
 
+@pytest.mark.parametrize("k,splits,stages", [(512, 1, 2), (1024, 1, 2), (1024, 2, 2), (1536, 1, 4), (1536, 2, 2),
+                                             (2560, 2, 4), (2048, 2, 2)])
+def test_qmm_short_q8_slices(torch_gpu, monkeypatch, k, splits, stages):
+    """Q8 of group size 32 on 128-row tiles: two activation stages while the
+    longest K slice has at most 16 steps (1024 k), four above."""
+    monkeypatch.setenv("MLXQ_QMM_CFG", "42")
+    monkeypatch.setenv("MLXQ_QMM_SPLIT", str(splits))
+    monkeypatch.setenv("MLXQ_QMM_FUSED", "1")
+    m, n = 200, 300
+    name = mlxq.qmatmul_route(m, n, k, 32, 8, algo=mlxq.ALGO_QMM)
+    assert name.startswith("qmm_short_kernel<8, 32, 4, 2>" if stages == 2 else "qmm_kernel<8, 32, 4, 2>"), name
+    wq, s, b = make_layer(0x71 + k, n, k, 32, 8)
+    x = bf16_acts(0x72, m, k)
+    y = run(x, wq, s, b, 32, 8, mlxq.ALGO_QMM)
+    assert rel_err(y, orc.qmatmul_f64(x, wq, s, b, 32, 8)) <= TIGHT
+
+
 @pytest.mark.parametrize("bits,m,n,k", [(4, 40, 5592405, 1536), (8, 40, 8388607, 512), (4, 1398101, 72, 1536),
                                         (4, 40, 5, 512), (8, 33, 9, 512)])
 def test_qmm_operands_just_below_4_gib(torch_gpu, bits, m, n, k):
