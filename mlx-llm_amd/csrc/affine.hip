@@ -57,7 +57,9 @@ __device__ __forceinline__ float load1(const void* p, int64_t i) {
 // enough elements: every lane of a group repeats it, so bf16 takes 16
 // elements per lane (14336 x 4096, Q4 / Q8: 45.9 / 45.8 us with 8 elements
 // and the general division, 36.3 / 37.5 with the shorter quotient, 29.6 /
-// 33.1 = 5.1 / 5.4 TB/s with 16).  f32 input is bound by its loads and takes
+// 33.1 = 5.1 / 5.4 TB/s with 16; those copies come from HBM in turn, a single
+// one repeated stays partly in the 256 MB cache: 23.9 / 26.0 against 28.5 /
+// 32.3).  f32 input is bound by its loads and takes
 // 8 (Q4 51 -> 47.9 us; 49.7 with 16, whose loads cover a quarter of each
 // line per instruction).  Two and four runs of lanes per workgroup measured
 // slower (bf16 Q4 30.9, f32 Q4 51.3 us with two).
@@ -92,7 +94,9 @@ __global__ __launch_bounds__(kThreads) void affine_quantize_kernel(const void* _
 // non-temporal and leave the caches to the codes: 14336 x 4096, bf16 Q4 / Q8
 // 31.0 / 35.0 -> 22.5 / 33.0 us, f32 Q4 / Q8 54.4 / 56.3 -> 39.2 / 52.9 (U =
 // 4: 22.8 / 32.5, 39.3 / 54.1; plain stores at U = 2: 30.7 / 34.2, 56.4 /
-// 53.9).
+// 53.9), on copies that come from HBM in turn; a single one repeated, whose
+// codes the non-temporal stores leave in the cache, takes 22.2 / 26.3, 39.2 /
+// 42.7.
 template <int DT, int BITS, int U>
 __global__ __launch_bounds__(kThreads) void affine_dequantize_kernel(const uint32_t* __restrict__ wq,
                                                                       const void* __restrict__ scales,

@@ -3,14 +3,15 @@
 // Reference: src/gguf/dequant.rs:156-211 (dispatcher) and the per-type block
 // decoders it calls (:228-719).  The reference walks blocks one at a time on
 // one host thread; here a workgroup stages a chunk of whole blocks into LDS
-// with wide coalesced loads, then every thread decodes VEC consecutive output
-// elements straight from LDS and writes them with one 16-byte store.
+// with wide coalesced loads, then every thread decodes runs of consecutive
+// output elements straight from LDS (8 for bf16, two of 4 for f32) and writes
+// each run with one 16-byte store.
 //
 // Bit-exactness: each output element is computed with exactly the IEEE f32
-// operations, operand order and roundings the reference uses for it (the
-// per-element formulas below are the reference's block loops solved for one
-// element).  This file is compiled with -ffp-contract=off so no mul+add/sub is
-// fused, and f16 scales are decoded with integer bit operations.
+// operations, operand order and roundings the reference uses for it
+// (gguf_decode.hpp).  This file is compiled with -ffp-contract=off so no
+// mul+add/sub is fused; f16 scales are converted by v_cvt_f32_f16, exact for
+// every encoding.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
