@@ -154,7 +154,8 @@ def test_qmatmul_add_rms_norm_graph_replay(torch_gpu):
     torch.cuda.synchronize()
     s_eager, y_eager = s_out.clone(), y_out.clone()
     g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g):
+    st = torch.cuda.Stream()  # its workspace is the graph's
+    with torch.cuda.graph(g, stream=st):
         mlxq.qmatmul_add_rms_norm(x, wd, sd, bd, r, w, 1e-5, 64, 4, sum_out=s_out, out=y_out)
     other = make_layer(704, 4096, 14336, 64, 8)
     od = (dev(other[0]), dev(other[1], True), dev(other[2], True))
@@ -164,5 +165,6 @@ def test_qmatmul_add_rms_norm_graph_replay(torch_gpu):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(s_out, s_eager) and torch.equal(y_out, y_eager), i
-        mlxq.qmatmul(x, *od, 64, 8)  # eager work through the same workspace
+        with torch.cuda.stream(st):
+            mlxq.qmatmul(x, *od, 64, 8)  # eager work through the same workspace
         torch.cuda.synchronize()

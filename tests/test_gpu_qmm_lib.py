@@ -109,7 +109,8 @@ def test_lib_graph_replay_bit_exact(torch_gpu, lib_all):
     eager = call().clone()
     torch.cuda.synchronize()
     g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g):
+    st = torch.cuda.Stream()  # its workspace is the graph's
+    with torch.cuda.graph(g, stream=st):
         call()
     other = make_layer(352, 768, 4096, 64, 8)
     od = [dev(other[0]), dev(other[1], bf16=True), dev(other[2], bf16=True)]
@@ -118,7 +119,8 @@ def test_lib_graph_replay_bit_exact(torch_gpu, lib_all):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(call.out, eager), i
-        mlxq.qmatmul(x, *od, 64, 8)  # another weight through the same workspace
+        with torch.cuda.stream(st):
+            mlxq.qmatmul(x, *od, 64, 8)  # another weight through the same workspace
         torch.cuda.synchronize()
 
 

@@ -207,14 +207,16 @@ def test_stream_graph_replay_bit_exact(torch_gpu, stream):
     torch.cuda.synchronize()
     eager = y.clone()
     g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g):
+    st = torch.cuda.Stream()  # its workspace is the graph's
+    with torch.cuda.graph(g, stream=st):
         call()
     for i in range(3):
         y.zero_()
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, eager), i
-        mlxq.qmatmul(xd, wd, sd, bd, 64, 4)  # eager work on the same workspace in between
+        with torch.cuda.stream(st):
+            mlxq.qmatmul(xd, wd, sd, bd, 64, 4)  # eager work on the same workspace in between
         torch.cuda.synchronize()
 
 

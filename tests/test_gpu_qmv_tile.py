@@ -138,14 +138,16 @@ def test_tile_graph_replay(torch_gpu, tile_all):
     e = c().clone()
     torch.cuda.synchronize()
     g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g):
+    st = torch.cuda.Stream()  # its workspace is the graph's
+    with torch.cuda.graph(g, stream=st):
         c()
     for i in range(4):
         c.out.zero_()
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(c.out, e), f"replay {i}"
-        mlxq.qmatmul(x[:8], *d, 64, 4)
+        with torch.cuda.stream(st):
+            mlxq.qmatmul(x[:8], *d, 64, 4)
         torch.cuda.synchronize()
 
 
